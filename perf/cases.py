@@ -55,8 +55,8 @@ def listed():
         # 3D variable density, orders 8 and 16 (the profiled workloads)
         _case(name="device-3d-vd-so8-256", nz=256, nx=256, ny=256, h=12.5, vd=True, nb=10,
               steps=100),
-        _case(name="device-3d-vd-so16-251", nz=251, nx=251, ny=251, h=12.5, vd=True, nb=10,
-              steps=100),
+        _case(name="device-3d-vd-so16-251", nz=251, nx=251, ny=251, h=12.5, so=16, vd=True,
+              nb=10, steps=100),
         # 3D variable density over a survey area that is longer than wide
         _case(name="device-3d-vd-so4-oblong", nz=120, nx=160, ny=231, vd=True, so=4, nb=20,
               steps=100),
