@@ -145,10 +145,12 @@ constexpr unsigned kAdjTimeUpdate = 8u;
 // before they are added to the float64 gradient
 constexpr size_t kGradFlush = 16;
 constexpr int kMaxFusedSources = 64;
-// cooperative receiver kernel: receivers per block and points per round
-// (LDS = kRecChunk * (kRecPerBlock + 1) values)
-constexpr int kRecPerBlock = sizeof(real_t) == 4 ? 16 : 8;
-constexpr int kRecChunk = 768;
+// cooperative receiver kernel: receivers per block and points per round (LDS:
+// about kRecPerBlock * kRecChunk values, 25 KB in 3D and 9 KB in 2D, so that
+// several blocks share a CU).  A round holds the box of the default window
+// (half-width 4: up to 9 points per axis); 3D float64 takes it in two.
+constexpr int kRecPerBlock = SW_DIM == 3 ? 8 : (sizeof(real_t) == 4 ? 16 : 8);
+constexpr int kRecChunk = SW_DIM == 2 ? 128 : (sizeof(real_t) == 4 ? 768 : 384);
 // grids from this many points on run the receiver gather on a second stream
 constexpr long long kOverlapMinPoints = 1ll << 22;
 
@@ -1059,10 +1061,7 @@ void launch_fused(const Params &P, const real_t *uc, const real_t *up, real_t *u
 }
 
 // k_step2d_z with the receiver gather of level n in the same launch (the
-// 2D z-marching path with receivers on the step stream); 64-product rounds
-// keep the gather's LDS at about 4 KB per block.
-constexpr int kRecChunkFused = 64;
-
+// 2D z-marching path with receivers on the step stream).
 template <int R>
 void launch_fused_rec(const Params &P, const real_t *uc, const real_t *up, real_t *un, int n,
                       hipStream_t st, LaunchTimer tm, const Box *rbox, const real_t *rw,
@@ -1073,7 +1072,7 @@ void launch_fused_rec(const Params &P, const real_t *uc, const real_t *up, real_
     const int zlen = zlen_2d(P, R);
     const int gz = (Iz + zlen - 1) / zlen;
     const int nrb = (nrec + kRecPerBlock - 1) / kRecPerBlock;
-    launch_timed(sw::k_step2d_z_rec<R, kRecPerBlock, kRecChunkFused>,
+    launch_timed(sw::k_step2d_z_rec<R, kRecPerBlock, kRecChunk>,
                  dim3((unsigned)(nrb + gx * gz)), dim3(sw::kZ2Block), st, tm, P, uc, up, un, n,
                  zlen, gx, nrb, rbox, rw, nrec, row);
 }
@@ -1093,7 +1092,7 @@ template <int R>
 void launch_persist(const Params &P, real_t *u, long long np, int n0, int n1, hipStream_t st,
                     const Box *rbox, const real_t *rw, int nrec, real_t *rec0, unsigned *bar)
 {
-    const auto kernel = sw::k_step2d_persist<R, kRecPerBlock, kRecChunkFused>;
+    const auto kernel = sw::k_step2d_persist<R, kRecPerBlock, kRecChunk>;
     static int per_cu = -1, ncu = 0;
     static std::mutex mu;
     {
