@@ -956,16 +956,17 @@ void setup_tiling(Prepared &pr, DeviceArena &arena, hipStream_t st)
     if (blocks >= (1ll << 31))
         return;
     T.nwords = P.nz / 32 + 3;
-    unsigned *mask = arena.alloc<unsigned>((size_t)T.ncols * T.nwords);
+    const long long words = (long long)T.ncols * T.nwords + 1;   // + den_bad
+    unsigned *mask = arena.alloc<unsigned>((size_t)words);
     {
-        const long long words = (long long)T.ncols * T.nwords;
         hipLaunchKernelGGL(sw::k_zero_u32,
                            dim3((unsigned)std::min<long long>((words + 255) / 256, 4096)),
                            dim3(256), 0, st, mask, words);
     }
     T.dmask = mask;
     hipLaunchKernelGGL(sw::k_damp_flags, dim3(T.ncols, P.nz), dim3(256), 0, st, P.e, P.nz,
-                       P.nx, P.ny, R, T.gk, T.ty, T.txr, T.nwords, mask);
+                       P.nx, P.ny, R, T.gk, T.ty, T.txr, T.nwords, mask,
+                       mask + words - 1);
     hip_check(hipGetLastError(), "k_damp_flags launch");
     Params *Pd = arena.alloc<Params>(1);
     hip_check(hipMemcpyAsync(Pd, &P, sizeof(Params), hipMemcpyHostToDevice, st),

@@ -54,7 +54,9 @@ struct Tiling {
     int chunk;          // columns per XCD chunk (order 1)
     int nwords;         // 32-bit mask words per tile column (nz/32 + 3)
     const unsigned *dmask;  // [ncols][nwords]: bit z set where plane z of the
-                            // tile column holds a non-zero damping term
+                            // tile column holds a non-zero damping term; then
+                            // one word, non-zero where some damped point's
+                            // den = 1 + e is outside recip_f64's range
 };
 
 // Sources restricted to the tile's mask, in index order (the reference's
@@ -84,7 +86,8 @@ __device__ __forceinline__ real_t add_sources_masked(const Params &P, int n, int
 // mask words must be zeroed beforehand.
 __global__ void __launch_bounds__(256)
 k_damp_flags(const real_t *__restrict__ e, int nz, int nx, int ny, int R, int gk,
-             int ty, int txr, int nwords, unsigned *__restrict__ mask)
+             int ty, int txr, int nwords, unsigned *__restrict__ mask,
+             unsigned *__restrict__ den_bad)
 {
     const int col = blockIdx.x, z = blockIdx.y;
     const int kt = col % gk, jt = col / gk;
@@ -92,12 +95,21 @@ k_damp_flags(const real_t *__restrict__ e, int nz, int nx, int ny, int R, int gk
     int any = 0;
     for (int t = threadIdx.x; t < ty * txr; t += blockDim.x) {
         const int k = k0 + t % ty, j = j0 + t / ty;
-        if (k < ny && j < nx)
-            any |= e[((long long)z * nx + j) * ny + k] != (real_t)0;
+        if (k < ny && j < nx) {
+            const real_t v = e[((long long)z * nx + j) * ny + k];
+            if (v != (real_t)0) {
+                const double den = fabs((double)(real_t)(1.0 + (double)v));
+                any |= den >= 0x1p-60 && den <= 0x1p60 ? 1 : 3;
+            }
+        }
     }
-    any = __syncthreads_or(any);
-    if (threadIdx.x == 0 && any)
+    const int damped = __syncthreads_or(any);
+    const int bad = __syncthreads_or(any & 2);
+    if (threadIdx.x == 0 && damped) {
         atomicOr(&mask[(long long)col * nwords + (z >> 5)], 1u << (z & 31));
+        if (bad)
+            atomicOr(den_bad, 1u);
+    }
 }
 
 // Bits z0 .. z0+63 of a tile column's damping mask.
@@ -182,19 +194,39 @@ __device__ __forceinline__ real_t leapfrog_damped(real_t value, real_t C, real_t
     return (real_t)t;
 }
 
+// RN(1/d) in float64 for a float d with 2^-60 <= |d| <= 2^60: a float32
+// reciprocal (relative error below 2^-22) and two Newton steps with fused
+// residuals.  After the first step 1 - d y is below 2^-43 and, d having 24
+// significant bits and y 53, a multiple of 2^-76: the second residual r is
+// exact, and y (1 + r) before its rounding is within 2^-86 of 1/d.  1/d lies
+// at least 2^-77 (relative) from every midpoint m between doubles (1 - d m
+// is a non-zero multiple of 2^-77 at that scale), so the rounding is that of
+// 1/d.  7 instructions instead of the 12 of the general float64 division.
+__device__ __forceinline__ double recip_f64(float d)
+{
+    const double b = (double)d;
+    double y = (double)__builtin_amdgcn_rcpf(d);
+    double r = __builtin_fma(-b, y, 1.0);
+    y = __builtin_fma(y, r, y);
+    r = __builtin_fma(-b, y, 1.0);
+    return __builtin_fma(y, r, y);
+}
+
 // The same update in float32 with one correctly rounded float64 reciprocal
 // y = RN(1/den) for the two quotients: RN(2/den) = 2y exactly, and for float
 // operands num/den (a normal quotient), rounding num*y first to double and
 // then to float gives RN(num/den): the product is within 2^-52 of the
 // quotient, and a quotient of two floats that is not a float lies at least
 // 2^-49 (relative) from every midpoint between floats.
+// FAST: den lies in recip_f64's range (k_damp_flags looks at every one).
+template <bool FAST>
 __device__ __forceinline__ float leapfrog_damped_rcp(float value, float C, float e,
                                                      float uc, float up)
 {
     const float den = (float)(1.0 + (double)e);
     const float num = (float)(1.0 - (double)e);
     value = value * C;
-    const double y = 1.0 / (double)den;
+    const double y = FAST ? recip_f64(den) : 1.0 / (double)den;
     const double a = 2.0 * y;
     const float b = (float)((double)num * y);
     double t = a * (double)uc - (double)(b * up);
@@ -425,6 +457,7 @@ k_step3d_vec(StepArgs A, const Params *__restrict__ Pd, int n)
     // update has consumed them.
     vreal nc[RPT], np[RPT], nq[RPT], ne[RPT], nhx[HX], nhy[HY];
     const unsigned long long dbits = damp_bits(T, col, z0);
+    const bool den_ok = T.dmask[(long long)T.ncols * T.nwords] == 0;
     auto load_centre = [&](int I) {
         const unsigned sp = (unsigned)(I - zb) * PB;   // plane I
         const unsigned vc = (unsigned)(I + R - zb) * PB;
@@ -619,16 +652,43 @@ k_step3d_vec(StepArgs A, const Params *__restrict__ Pd, int n)
             for (int e = 0; e < V; e++) {
                 real_t value = 0;
                 value += lap[e];
-#if defined(SW_DOUBLE)
-                out[q][e] = damped ? leapfrog_damped(value, nq[q][e], ne[q][e], qz[q][R][e],
-                                                     np[q][e])
-                                   : leapfrog_plain(value, nq[q][e], qz[q][R][e], np[q][e]);
-#else
-                out[q][e] = damped ? leapfrog_damped_rcp(value, nq[q][e], ne[q][e],
-                                                         qz[q][R][e], np[q][e])
-                                   : leapfrog_plain(value, nq[q][e], qz[q][R][e], np[q][e]);
-#endif
+                out[q][e] = value;
             }
+        }
+        // The update operands are first touched here, after every row's
+        // stencil: one uniform branch over all points, behind a scheduling
+        // barrier, so that their loads have the whole stencil to arrive (a
+        // branch per point, folded into the stencil, waited for them at the
+        // start of the plane).
+        __builtin_amdgcn_sched_barrier(0);
+        auto update = [&](auto f) {
+#pragma unroll
+            for (int q = 0; q < RPT; q++)
+#pragma unroll
+                for (int e = 0; e < V; e++)
+                    out[q][e] = f(out[q][e], nq[q][e], ne[q][e], qz[q][R][e], np[q][e]);
+        };
+        if (!damped)
+            update([](real_t v, real_t C, real_t, real_t uc, real_t up) {
+                return leapfrog_plain(v, C, uc, up);
+            });
+#if defined(SW_DOUBLE)
+        else
+            update([](real_t v, real_t C, real_t e, real_t uc, real_t up) {
+                return leapfrog_damped(v, C, e, uc, up);
+            });
+#else
+        else if (den_ok)
+            update([](real_t v, real_t C, real_t e, real_t uc, real_t up) {
+                return leapfrog_damped_rcp<true>(v, C, e, uc, up);
+            });
+        else
+            update([](real_t v, real_t C, real_t e, real_t uc, real_t up) {
+                return leapfrog_damped_rcp<false>(v, C, e, uc, up);
+            });
+#endif
+#pragma unroll
+        for (int q = 0; q < RPT; q++) {
             if (!CLEAN && special && act[q]) {
                 // tiles touching a source box or a boundary face
                 const int j = j0 + slot * RPT + q;
