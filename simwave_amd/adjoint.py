@@ -64,7 +64,7 @@ def _run(dev, rec_adjoint, checkpoint_every, want_wavelet, stream=None, image=Fa
     kw = dev.kwargs
     checkpoint_every = checkpoint_interval(dev, checkpoint_every)
     lib = dev._lib
-    fn = getattr(lib, "simwave_hip_gradient_" + dev.variant)
+    fn = lib["simwave_hip_gradient_" + dev.variant]
     fn.restype = ctypes.c_double
     fn.argtypes = list(dev._argtypes) + [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                          ctypes.c_size_t, ctypes.c_void_p, ctypes.c_uint]

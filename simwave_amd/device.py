@@ -100,7 +100,10 @@ class DeviceForward:
             density=kwargs.get("density_model"),
             dtype=kwargs["velocity_model"].dtype)
         self._lib = lib
-        self._fn = getattr(lib, "simwave_hip_forward_device_" + self.variant)
+        # function objects of this shot's own (lib[name], not the cached
+        # lib.name): shots are built on several threads, and argtypes set on
+        # a shared object would be freed under another thread's call
+        self._fn = lib["simwave_hip_forward_device_" + self.variant]
         st = self._stream(stream)
         keep = []           # host arrays of copies still in flight
         self.tensors = {}
@@ -139,21 +142,21 @@ class DeviceForward:
         self._fn.restype = ctypes.c_double
         self._fn.argtypes = argtypes + [ctypes.c_void_p, ctypes.c_uint]
         self._args = args
-        self._plan_create = getattr(lib, "simwave_hip_plan_create_" + self.variant)
+        self._plan_create = lib["simwave_hip_plan_create_" + self.variant]
         self._plan_create.restype = ctypes.c_void_p
         self._plan_create.argtypes = argtypes + [ctypes.c_void_p, ctypes.c_uint]
-        self._plan_run = getattr(lib, "simwave_hip_plan_run_" + self.variant)
+        self._plan_run = lib["simwave_hip_plan_run_" + self.variant]
         self._plan_run.restype = ctypes.c_longlong
         self._plan_run.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
-        self._plan_destroy = getattr(lib, "simwave_hip_plan_destroy_" + self.variant)
+        self._plan_destroy = lib["simwave_hip_plan_destroy_" + self.variant]
         self._plan_destroy.restype = ctypes.c_int
         self._plan_destroy.argtypes = [ctypes.c_void_p]
-        self._plans_run = getattr(lib, "simwave_hip_plans_run_" + self.variant)
+        self._plans_run = lib["simwave_hip_plans_run_" + self.variant]
         self._plans_run.restype = ctypes.c_int
         self._plans_run.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_int,
                                     ctypes.c_size_t, ctypes.c_void_p,
                                     ctypes.POINTER(ctypes.c_longlong)]
-        self._plan_batchable = getattr(lib, "simwave_hip_plan_batchable_" + self.variant)
+        self._plan_batchable = lib["simwave_hip_plan_batchable_" + self.variant]
         self._plan_batchable.restype = ctypes.c_int
         self._plan_batchable.argtypes = [ctypes.c_void_p]
         self._plan = None
@@ -215,7 +218,7 @@ class DeviceForward:
         keep.extend([src] + idx)
         shape = tuple(len(i) for i in index)
         out = self._empty(shape, small.dtype, stream)
-        fn = getattr(self._lib, "simwave_hip_gather_" + self.variant)
+        fn = self._lib["simwave_hip_gather_" + self.variant]
         fn.restype = ctypes.c_int
         fn.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int,
                        ctypes.POINTER(ctypes.c_longlong), ctypes.POINTER(ctypes.c_longlong),
@@ -352,7 +355,7 @@ class DeviceForward:
         [total s, prepare s, loop s, download s, step-kernel s, step launches,
          fused(1)/generic(0), step kernel: 3D tiled(1)/z-marching(2)/other(0)]."""
         out = (ctypes.c_double * 8)()
-        fn = self._lib.simwave_hip_last_timings
+        fn = self._lib["simwave_hip_last_timings"]
         fn.argtypes = [ctypes.POINTER(ctypes.c_double), ctypes.c_int]
         fn.restype = ctypes.c_int
         fn(out, 8)

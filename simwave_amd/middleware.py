@@ -112,7 +112,9 @@ class Middleware:
                            density=kwargs.get("density_model"),
                            dtype=vel.dtype)
         argtypes, args = self.ordered(kwargs)
-        fn = lib.forward
+        # a function object of this call's own: argtypes set on the cached
+        # lib.forward would be freed under another thread's call
+        fn = lib["forward"]
         fn.restype = ctypes.c_double
         fn.argtypes = argtypes
         seconds = fn(*args)
@@ -136,7 +138,7 @@ class Middleware:
 
 def _last_error(lib):
     try:
-        fn = lib.simwave_hip_last_error
+        fn = lib["simwave_hip_last_error"]
     except AttributeError:
         return None
     fn.restype = ctypes.c_char_p
