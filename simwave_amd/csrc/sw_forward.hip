@@ -382,9 +382,10 @@ struct Prepared {
     void (*tiled_launch)(const struct Prepared &, const real_t *, const real_t *,
                          real_t *, int, hipStream_t, LaunchTimer) = nullptr;
     const Params *Pd = nullptr;   // device copy of P for the tiled kernel
-    const real_t *qc = nullptr;   // (dt2/s)/den per point for the tiled kernel
+    const real_t *pk = nullptr, *pe = nullptr;   // its packed coefficients (k_pack_tiles)
     bool fastdiv = false;
     bool div64 = false;          // float64-reciprocal quotients in the tiled kernel
+    bool div64_check = false;    // ... whose subnormal results need IEEE division
     sw::FixedDiv dvz{}, dvx{}, dvy{};
     sw::Tiling tiling{};
     int tiled_blocks = 0;
@@ -394,6 +395,7 @@ struct Prepared {
 #if SW_DIM == 3
 void setup_tiling(Prepared &pr, DeviceArena &arena, hipStream_t st);
 bool prefer_zmarch(const Prepared &pr);
+bool prefer_tiled_vd(const Prepared &pr, bool oblong, const DeviceArena &arena);
 void set_lap_div(Prepared &pr);
 #else
 bool zmarch_2d(int R);
@@ -597,10 +599,6 @@ Prepared prepare(const Args &a, bool dev_models, unsigned flags,
             fused = false;
     if (a.nsrc > (size_t)kMaxFusedSources)
         fused = false;
-#if SW_DIM == 3 && SW_VD
-    if (a.nx != a.ny)
-        fused = false;
-#endif
     pr.fused = fused;
 #if SW_DIM == 3 && !SW_VD
     // the z-marching one-point-per-thread kernel where it is the faster one
@@ -619,12 +617,21 @@ Prepared prepare(const Args &a, bool dev_models, unsigned flags,
         }
     }
 #elif SW_DIM == 3
-    // variable density: the z-marching kernel where it is the faster one
-    // (prefer_zmarch) or when asked for; the LDS-tiled k_step3d otherwise.
+    // variable density: the tiled kernel where it is the faster one
+    // (prefer_tiled_vd) or when asked for (SIMWAVE_HIP_TILE); the z-marching
+    // kernel where that one is (prefer_zmarch) or when asked for; the
+    // LDS-tiled k_step3d otherwise.  With nx != ny only the tiled kernel has
+    // the reference's x-axis stride: the generic kernels run where it does
+    // not fit.
     // Its z chunks: 16 planes, halved (down to 4) while the launch holds
     // fewer than 2048 blocks (448^3 so8: 854 us at 16 planes, 894 at 8;
     // 176^3 so8: 65 us at 4 planes, 71 at 16)
-    if (fused && !env_flag("SIMWAVE_HIP_UNTILED") &&
+    const bool oblong = a.nx != a.ny;
+    if (fused && prefer_tiled_vd(pr, oblong, arena))
+        setup_tiling(pr, arena, st);
+    if (oblong && !pr.tiled)
+        fused = pr.fused = false;
+    if (fused && !pr.tiled && !env_flag("SIMWAVE_HIP_UNTILED") &&
         (env_flag("SIMWAVE_HIP_ZMARCH") || prefer_zmarch(pr))) {
         pr.zmarch = true;
         int zl = env_int("SIMWAVE_HIP_ZLEN", 0);
@@ -642,11 +649,11 @@ Prepared prepare(const Args &a, bool dev_models, unsigned flags,
 #endif
 #if SW_VD
 #if SW_DIM == 3
-    const bool zm = pr.zmarch;
+    const bool pre = pr.zmarch && r >= sw::kVdPre;
 #else
-    const bool zm = fused && zmarch_2d(r);
+    const bool pre = fused && zmarch_2d(r) && r >= sw::kVdPre;
 #endif
-    if (zm && r >= sw::kVdPre)
+    if (pre)
         rho_diff(pr, arena, st);
 #endif
     return pr;
@@ -700,13 +707,19 @@ bool make_fixed_div(real_t b, sw::FixedDiv &d)
 // lies at least 2^-48 from the midpoints (2j+1) 2^-150: with t <= 0,
 // (2j+1) B 2^(t-150) is an odd multiple of 2^(t-150) and a is a multiple
 // of 2^-149, so they differ.  Both separations exceed the product's error.
+// f64_quotient_near: without t <= 0, where that holds for every a whose
+// quotient is normal or zero.
+bool f64_quotient_near(real_t b)
+{
+    return sizeof(real_t) == 4 && (double)b >= std::ldexp(1.0, -126) &&
+           (double)b < std::ldexp(1.0, 24);
+}
+
 bool f64_quotient_exact(real_t b)
 {
-    if (sizeof(real_t) != 4)
+    if (!f64_quotient_near(b))
         return false;
     const double bd = (double)b;
-    if (!(bd >= std::ldexp(1.0, -126) && bd < std::ldexp(1.0, 24)))
-        return false;
     int e = 0;
     const double m = std::frexp(bd, &e);              // bd = m 2^e, m in [0.5, 1)
     unsigned long long S = (unsigned long long)std::ldexp(m, 24);   // 24-bit significand
@@ -734,69 +747,104 @@ void set_lap_div(Prepared &pr)
 
 #if SW_DIM == 3
 // Tile configurations of k_step3d_vec as (rows per wavefront WR, rows per
-// thread RPT, wavefronts per block NW, and 16- or 8-byte lanes).  Radius 4
-// (space order 8) carries every configuration; other radii carry 0, 4, 8,
-// 17 and 18.  SIMWAVE_HIP_TILE picks one; otherwise default_tile().
-// Measured per launch on one MI355X, float32, radius 4, 6-plane z chunks:
-//  * spacings whose Laplacian quotients are float64 products (div64):
-//    8 rows x 64 points of 8-byte lanes with 4 rows per lane are fastest,
-//    1-3% ahead of the same tile of 16-byte lanes with 2 rows per lane
-//    (472^3: 515 against 532 us; interior 340^3 245 against 248, 380^3 318
-//    against 322, 420^3 411 against 420; 300^3 even).  The 8-byte lanes halve the registers of a z
-//    queue entry, so a lane holds 4 adjacent rows and takes more of its x
-//    neighbours from registers.  The 4 x 128 shape of 8-byte lanes was
-//    fastest at 472^3 alone (511 us) and 2-8% behind elsewhere; shapes with
-//    3 wavefronts per SIMD (133-137 VGPRs) came to 541-578 us at 472^3.
-//  * other spacings (fixed-divisor quotients): the 16-byte 8 x 64 tile, the
-//    8-byte one within 2% either way (300^3-380^3 interior), 5% behind at
-//    260^3.
-// Radii 5-10: 8 rows x 32 points of 16-byte lanes and 4-plane chunks
-// (10-13% ahead of 4-wavefront tiles at 312^3-376^3; the 8-byte shapes
-// 1-10% behind at 320^3 so12 and so16).  Float64: 8 rows x 32 points of
-// 16-byte lanes, 8-plane chunks at radius 4 (472^3: 881 us; the 8-byte
-// shapes 894-1097 us), 12-plane chunks elsewhere.
+// thread RPT, wavefronts per block NW, and 16- or 8-byte lanes).  Constant
+// density: radius 4 (space order 8) carries every configuration, other radii
+// 0, 4, 8, 17 and 18; SIMWAVE_HIP_TILE picks one, otherwise default_tile().
+// Variable density carries one shape per radius (tiled_entry).
+// Measured per launch on one MI355X with the packed coefficients:
+//  * float32 radius 4: 8 rows x 64 points of 8-byte lanes with 4 rows per
+//    lane (17) for large grids (472^3: 502 us, the same tile of 16-byte lanes
+//    with 2 rows per lane (10) 526; 216 x 316 x 316 interior: 136 each), the
+//    16-byte tile below 20 M interior points (240^3: 88 against 90 us).
+//  * float32 radius 3: 17 (340^3: 228 us, 8: 252).  Radii 5-10: 8 rows x 32
+//    points of 16-byte lanes (8): 240^3 so16 97 us (17: 107), so20 116 (122);
+//    241 x 317 x 341 so12 176 (174).
+//  * float64: radius 4 the 16-byte 8 x 32 tile (10: 221 x 243 x 259 152 us, 17
+//    153, 8 173); below, 8 x 16 points with 2 rows per lane (18: 240^3 so4
+//    142, 17 147, 4 158); radii 5-7 four wavefronts (4: so12 157, 8 175);
+//    above, one (8: so16 168, 4 176).
 constexpr int kTileShapes = 24;
-constexpr int default_tile(int R, bool div64)
+// scratch left to the small tables behind the packed coefficients
+constexpr size_t kPackSlack = 1u << 20;
+constexpr bool kF32 = sizeof(real_t) == 4;
+
+int default_tile(int R, bool div64, long long interior)
 {
-    return R == 4 ? (sizeof(real_t) == 4 && div64 ? 17 : 10)
-         : R < 4 ? 0 : (sizeof(real_t) == 4 ? 8 : 4);
-}
-constexpr int default_tile_zlen(int R)
-{
-    return sizeof(real_t) == 4 ? (R == 4 ? 6 : R > 4 ? 4 : 12) : (R == 4 ? 8 : 12);
+    if (SW_VD)
+        return 0;
+    if (kF32)
+        return R == 4 ? (div64 && interior >= 20ll * 1000 * 1000 ? 17 : 10) : R < 4 ? 17 : 8;
+    return R == 4 ? 10 : R < 4 ? 18 : R < 8 ? 4 : 8;
 }
 
-// Whether the z-marching one-point-per-thread kernel beats the tiled one
-// for this grid.  Its 7 wavefronts per SIMD hide latency better while the
-// grid holds too few tiles to keep the tiled kernel's 2 per SIMD busy; its
-// neighbour reads through the caches lose once there are plenty at radius 4.
-// Measured per launch (float32, cubes): radius 1-3 at every size up to
-// 466^3 (1.2-1.9x faster than any tile configuration); radius 4 up to
-// ~30 M interior points (interior 260^3: 126 against 144 us; 300^3, 27 M:
-// 172 against 187 us, 198 us with float64-product quotients; 320^3, 33 M:
-// tiled 192 against 209 us; 384^3, 57 M: 327 against 347 us; with the
-// tiled kernel's 6-plane chunks and Dirichlet faces in its clean march);
-// radius 5+ never (its register queue is 2R+1 deep).
-// Float64: the tiled kernel (z-marching 26% slower at 22 M, radius 4).
-// Variable density: float32 at every radius and size measured, 1.2-1.8x
-// faster than the LDS-tiled k_step3d (176^3-448^3, orders 2-16); float64 at
-// radius <= 4 (272^3 so8: 527 vs 690 us; 268^3 so4: 346 vs 413 us), above
-// which its double-precision register queues would spill.
+// Planes per z chunk.  Short chunks: the tiles in flight on an XCD then cover
+// few planes and share their halo rows in its L2 (256^3 variable density so8:
+// 4 planes fetch 0.82 GB per step and take 185 us, 12 planes 212 us, 24
+// planes 1.02 GB); large grids and the long prologues of high orders want a
+// few more (472^3: 6 planes 502 us, 4 514; so16 float64 240^3: 12 planes 168,
+// 4 178), small grids fewer, to fill the chip (148^3 variable density so8: 2
+// planes 38.1 us, 4 40.0; 168^3 so16 42.3 and 43.9).
+int default_tile_zlen(int R, long long interior)
+{
+    if (interior < 5ll * 1000 * 1000)
+        return 2;
+    if (SW_VD)
+        return kF32 ? (R < 8 ? 4 : 6) : (R < 6 ? 4 : 8);
+    if (R == 4)
+        return interior < 30ll * 1000 * 1000 ? 4 : kF32 ? 6 : 8;
+    return kF32 || R < 8 ? 4 : 12;
+}
+
+long long interior_points(const Prepared &pr)
+{
+    const Params &P = pr.P;
+    const int R = pr.r;
+    return (long long)(P.nz - 2 * R) * (P.nx - 2 * R) * (P.ny - 2 * R);
+}
+
+// Constant density: whether the z-marching one-point-per-thread kernel runs.
+// Its 7 wavefronts per SIMD hide latency better while the grid holds too few
+// tiles to keep the tiled kernel's 2 per SIMD busy; its neighbour reads
+// through the caches lose once there are plenty.  Measured per launch
+// (float32, cubes of the interior size): radius 1-2 at every size (340^3 so2:
+// 203 against 235 us, so4 235 against 243); radius 3 (340^3) 255 against 228;
+// radius 4 168^3 41 against 46 us, 240^3 100 against 88, 216 x 316 x 316 148
+// against 136; radius 5+ never (its register queue is 2R+1 deep).  Float64:
+// the tiled kernel (240^3 so4: 155 against 142 us; so8 229 against 152).
+// Variable density, where the tiled kernel does not run: float32 always,
+// 1.2-1.8x faster than the LDS-tiled k_step3d (176^3-448^3, orders 2-16);
+// float64 at radius <= 4, above which its double-precision register queues
+// would spill.
 bool prefer_zmarch(const Prepared &pr)
 {
     if (SW_VD)
-        return sizeof(real_t) == 4 || pr.r <= 4;
-    if (sizeof(real_t) != 4)
+        return kF32 || pr.r <= 4;
+    if (!kF32 || pr.r > 4)
         return false;
-    const Params &P = pr.P;
-    const int R = pr.r;
-    const long long interior = (long long)(P.nz - 2 * R) * (P.nx - 2 * R) * (P.ny - 2 * R);
-    if (R <= 3)
-        return true;
-    return R == 4 && interior < 30ll * 1000 * 1000;
+    return pr.r <= 2 || interior_points(pr) < 8ll * 1000 * 1000;
 }
 
-template <int R, int WR, int RPT, int NW, int V, bool D64>
+// Variable density: whether the tiled kernel runs.  Always where nx != ny
+// (only it has the reference's x-axis stride; 160 x 200 x 271 so4: 92 us for
+// the whole step, the generic kernels 85 us for the stencil alone and 22 us
+// for sources and boundaries; so16 160 against 232 us).  Otherwise from 2 M
+// interior points on: float32 from radius 3 (276^3 so8: 185 us, z-marching
+// 275; so16 220 against 317; 148^3 so8 38 against 54; 116^3 29 against 30;
+// but 220^3 so2 100 against 80, so4 104 against 105), float64 from radius 2
+// (220^3 so4 170 against 227, so8 171 against 344, so16 234 against k_step3d's
+// 459).  A caller-owned arena (the allocation-free entry) has no room
+// for the packed coefficients.
+bool prefer_tiled_vd(const Prepared &pr, bool oblong, const DeviceArena &arena)
+{
+    if (!SW_VD || env_flag("SIMWAVE_HIP_UNTILED") || env_flag("SIMWAVE_HIP_ZMARCH") || arena.base)
+        return false;
+    const char *tile = getenv("SIMWAVE_HIP_TILE");
+    if ((tile && *tile) || oblong)
+        return true;
+    return pr.r >= (kF32 ? 3 : 2) && interior_points(pr) >= 2ll * 1000 * 1000;
+}
+
+template <int R, int WR, int RPT, int NW, int V, bool D64, int RHO>
 void tiled_launch(const Prepared &pr, const real_t *uc, const real_t *up, real_t *un,
                   int n, hipStream_t st, LaunchTimer tm)
 {
@@ -804,8 +852,8 @@ void tiled_launch(const Prepared &pr, const real_t *uc, const real_t *up, real_t
     sw::StepArgs A{};
     A.uc = uc;
     A.up = up;
-    A.qc = pr.qc;
-    A.e = P.e;
+    A.pk = pr.pk;
+    A.pe = pr.pe;
     A.un = un;
     A.fastdiv = pr.fastdiv ? 1 : 0;
     A.dvz = pr.dvz;
@@ -816,6 +864,14 @@ void tiled_launch(const Prepared &pr, const real_t *uc, const real_t *up, real_t
     A.ry = 1.0 / (double)P.dy2;
     A.rx = 1.0 / (double)P.dx2;
     A.rz = 1.0 / (double)P.dz2;
+    A.d64_check = pr.div64_check ? 1 : 0;
+    if constexpr (RHO != 0) {
+        A.r4y = 1.0 / (double)(4 * P.dy2);
+        A.r4x = 1.0 / (double)(4 * P.dx2);
+        A.r4z = 1.0 / (double)(4 * P.dz2);
+        for (int m = 0; m <= sw::kMaxR; m++)
+            A.c1[m] = P.c1[m];
+    }
     A.nz = P.nz;
     A.nx = P.nx;
     A.ny = P.ny;
@@ -831,7 +887,7 @@ void tiled_launch(const Prepared &pr, const real_t *uc, const real_t *up, real_t
     A.nsrc = P.nsrc;
     A.sbox = P.sbox;
     A.T = pr.tiling;
-    launch_timed(sw::k_step3d_vec<R, WR, RPT, NW, V, D64>, dim3(pr.tiled_blocks), dim3(64, NW),
+    launch_timed(sw::k_step3d_vec<R, WR, RPT, NW, V, D64, RHO>, dim3(pr.tiled_blocks), dim3(64, NW),
                  st, tm, A, pr.Pd, n);
 }
 
@@ -841,6 +897,8 @@ struct TiledKernel {
     TiledFn launch;
     TiledFn launch64;   // float64-reciprocal quotients (float32 builds)
     int ty, txr;
+    sw::PackShape pack;
+    TiledFn launch_q, launch64_q;   // variable density with nx != ny
 };
 
 template <int R, int WR, int RPT, int NW, int V = sw::kVec16>
@@ -848,13 +906,30 @@ TiledKernel tiled_config()
 {
     using S = sw::TileShape<R, WR, RPT, NW, V>;
     constexpr bool f32 = sizeof(real_t) == 4;
-    return TiledKernel{&tiled_launch<R, WR, RPT, NW, V, false>,
-                       &tiled_launch<R, WR, RPT, NW, V, f32>, S::TY, S::TXR};
+    TiledKernel K{&tiled_launch<R, WR, RPT, NW, V, false, SW_VD>,
+                  &tiled_launch<R, WR, RPT, NW, V, f32, SW_VD>, S::TY, S::TXR,
+                  {WR, RPT, 64 * NW, V}, nullptr, nullptr};
+#if SW_VD
+    K.launch_q = &tiled_launch<R, WR, RPT, NW, V, false, 2>;
+    K.launch64_q = &tiled_launch<R, WR, RPT, NW, V, f32, 2>;
+#endif
+    return K;
 }
 
 template <int R>
 TiledKernel tiled_entry(int v)
 {
+#if SW_VD
+    // 8 rows of 8-byte lanes with 2 rows per lane up to radius 5 (float64: 4),
+    // above it 8 rows of 16-byte lanes, whose one row per lane keeps the z
+    // queue short (276^3 so8: 185 against 196 us; so16 224 against 220, 220^3
+    // so20 200 against 191; float64 so16 257 against 234)
+    (void)v;
+    if constexpr (R <= (kF32 ? 5 : 4))
+        return tiled_config<R, 4, 2, 1, sw::kVec8>();
+    else
+        return tiled_config<R, 8, 1, 1, sw::kVec16>();
+#else
     if constexpr (R == 4) {
         switch (v) {
         case 1: return tiled_config<R, 1, 2, 4>();
@@ -890,6 +965,7 @@ TiledKernel tiled_entry(int v)
              : v == 18 ? tiled_config<R, 2, 2, 1, sw::kVec8>()
                        : tiled_config<R, 1, 1, 4>();
     }
+#endif
 }
 
 TiledKernel tiled_kernel(int R, int v)
@@ -915,13 +991,20 @@ void setup_tiling(Prepared &pr, DeviceArena &arena, hipStream_t st)
 {
     const Params &P = pr.P;
     const int R = pr.r;
-    // float32 Laplacian quotients as float64 products with RN(1/h^2)
-    // where that gives the IEEE quotient for every numerator
-    const bool div64 = sizeof(real_t) == 4 && !env_flag("SIMWAVE_HIP_IEEE_DIV") &&
-                       !env_flag("SIMWAVE_HIP_NO_DIV64") && f64_quotient_exact(P.dz2) &&
-                       f64_quotient_exact(P.dx2) && f64_quotient_exact(P.dy2);
-    int shape = env_int("SIMWAVE_HIP_TILE", default_tile(R, div64));
-    shape = shape >= 0 && shape < kTileShapes ? shape : default_tile(R, div64);
+    // float32 Laplacian quotients as float64 products with RN(1/h^2) where
+    // that gives the IEEE quotient for every numerator, or for all but
+    // subnormal quotients, which the kernel then looks for (241 x 317 x 341
+    // so12, h = 10: 176 us, fixed-divisor quotients with their range vote 179)
+    bool div64 = sizeof(real_t) == 4 && !env_flag("SIMWAVE_HIP_IEEE_DIV") &&
+                 !env_flag("SIMWAVE_HIP_NO_DIV64");
+    for (const real_t b : {P.dz2, P.dx2, P.dy2}) {
+        const bool exact = f64_quotient_exact(b) && (!SW_VD || f64_quotient_exact(4 * b));
+        div64 = div64 && f64_quotient_near(b) && (!SW_VD || f64_quotient_near(4 * b));
+        pr.div64_check = pr.div64_check || !exact;
+    }
+    const int dflt = default_tile(R, div64, interior_points(pr));
+    int shape = env_int("SIMWAVE_HIP_TILE", dflt);
+    shape = shape >= 0 && shape < kTileShapes ? shape : dflt;
     const TiledKernel K = tiled_kernel(R, shape);
     const int Iy = P.ny - 2 * R, Ix = P.nx - 2 * R, Iz = P.nz - 2 * R;
     const long long pbytes = (long long)P.nx * P.ny * (long long)sizeof(real_t);
@@ -937,13 +1020,9 @@ void setup_tiling(Prepared &pr, DeviceArena &arena, hipStream_t st)
     T.ncols = T.gk * T.gj;
     T.order = env_int("SIMWAVE_HIP_ORDER", 1) == 1 ? 1 : 0;
     T.chunk = (T.ncols + 7) / 8;
-    // short z chunks (default_tile_zlen planes): short tiles keep many
-    // independent blocks in every phase (prologue, march) on each CU, which
-    // overlaps their loads and arithmetic better than long marches, at
-    // 2R/zlen extra centre-plane reads
     int zlen = env_int("SIMWAVE_HIP_ZLEN", 0);
     if (zlen <= 0) {
-        const int target = default_tile_zlen(R);
+        const int target = default_tile_zlen(R, interior_points(pr));
         const int chunks = std::max(1, (Iz + target - 1) / target);
         zlen = (Iz + chunks - 1) / chunks;
     }
@@ -956,6 +1035,12 @@ void setup_tiling(Prepared &pr, DeviceArena &arena, hipStream_t st)
     if (blocks >= (1ll << 31))
         return;
     T.nwords = P.nz / 32 + 3;
+    // the packed coefficients; a caller-owned arena that cannot take them
+    // leaves the run to the other kernels
+    const size_t tile_points = (size_t)T.ncols * Iz * T.ty * T.txr;
+    if (arena.base && tile_points * (SW_VD ? 6 : 2) * sizeof(real_t) + kPackSlack >
+                          arena.cap - arena.used)
+        return;
     const long long words = (long long)T.ncols * T.nwords + 1;   // + den_bad
     unsigned *mask = arena.alloc<unsigned>((size_t)words);
     {
@@ -972,18 +1057,19 @@ void setup_tiling(Prepared &pr, DeviceArena &arena, hipStream_t st)
     hip_check(hipMemcpyAsync(Pd, &P, sizeof(Params), hipMemcpyHostToDevice, st),
               "copy params");
     pr.Pd = Pd;
-    {
-        real_t *qc = arena.alloc<real_t>(pr.npts);
-        const int nb = (int)std::min<long long>((pr.npts + 255) / 256, 8192);
-        hipLaunchKernelGGL(sw::k_scaled_q, dim3(nb), dim3(256), 0, st, P.q, P.e, qc,
-                           pr.npts);
-        hip_check(hipGetLastError(), "k_scaled_q launch");
-        pr.qc = qc;
-    }
+    real_t *pk = arena.alloc<real_t>(tile_points * (SW_VD ? 5 : 1));
+    real_t *pe = arena.alloc<real_t>(tile_points);
+    hipLaunchKernelGGL(sw::k_pack_tiles, dim3(T.ncols, Iz), dim3(256), 0, st, P, R, K.pack, T.gk,
+                       T.ty, T.txr, T.ncols, SW_VD, pk, pe);
+    hip_check(hipGetLastError(), "k_pack_tiles launch");
+    pr.pk = pk;
+    pr.pe = pe;
     pr.fastdiv = !env_flag("SIMWAVE_HIP_IEEE_DIV") && make_fixed_div(P.dz2, pr.dvz) &&
                  make_fixed_div(P.dx2, pr.dvx) && make_fixed_div(P.dy2, pr.dvy);
     pr.div64 = div64;
-    pr.tiled_launch = pr.div64 ? K.launch64 : K.launch;
+    const bool oblong = SW_VD && P.nx != P.ny;
+    pr.tiled_launch = pr.div64 ? (oblong ? K.launch64_q : K.launch64)
+                               : (oblong ? K.launch_q : K.launch);
     pr.tiling = T;
     pr.tiled_blocks = (int)blocks;
     pr.tiled = true;
@@ -2614,19 +2700,10 @@ double run_adjoint(const Args &a, const real_t *rec_adj, double *grad, real_t *g
     // the sums do not depend on K) and at the end they go into grad
     real_t *gacc = arena.alloc<real_t>(npts);
     size_t reverse_steps = 0;
-    // the forward's coefficient C = q / den per point (the tiled kernel's
-    // copy where it was built)
-#if SW_DIM == 3
-    const real_t *Cq = pr.qc;
-#else
-    const real_t *Cq = nullptr;
-#endif
-    if (!Cq) {
-        real_t *c = arena.alloc<real_t>(npts);
-        hipLaunchKernelGGL(sw::k_scaled_q, dim3(nb), dim3(256), 0, st, P.q, P.e, c,
-                           (long long)npts);
-        Cq = c;
-    }
+    // the forward's coefficient C = q / den per point
+    real_t *Cq = arena.alloc<real_t>(npts);
+    hipLaunchKernelGGL(sw::k_scaled_q, dim3(nb), dim3(256), 0, st, P.q, P.e, Cq,
+                       (long long)npts);
     auto flush_grad = [&]() {
         hipLaunchKernelGGL(sw::k_grad_flush, dim3(nb), dim3(256), 0, st, gacc, grad,
                            (long long)npts);

@@ -112,6 +112,61 @@ k_damp_flags(const real_t *__restrict__ e, int nz, int nx, int ny, int R, int gk
     }
 }
 
+// Lane layout of a tile, as k_step3d_vec's TileShape.
+struct PackShape {
+    int wr, rpt, nt, v;   // rows per wavefront, rows per lane, threads, points per vector
+};
+
+// The step-independent values of every interior point in the order the tiled
+// kernel reads them: per tile column and interior plane, per value (C =
+// (dt2/s)/den; with variable density then the density's derivative sums along
+// z, x and y and the density), per 16-byte chunk of a lane's points, all
+// threads' chunks.  A wavefront's loads are then whole aligned 1 KB runs
+// whatever the grid's row length: rows of a tile in the grid's own layout
+// are 256-byte pieces that straddle one more cache line than they fill
+// (4 rows of 256 bytes load at 5.3 TB/s from HBM, 1 KB runs at 7.0), and
+// 16-byte loads take the load path no longer than 8-byte ones.  pe: the
+// damping terms in the same order.  Values outside the interior are zero.
+// The sums are formed in the reference's order (vd-3d wave.c:175-186, where
+// the x axis steps by nx elements) from +0.
+__global__ void __launch_bounds__(256)
+k_pack_tiles(Params P, int R, PackShape S, int gk, int ty, int txr, int ncols, int rho,
+             real_t *__restrict__ pk, real_t *__restrict__ pe)
+{
+    const int lp = S.rpt * S.v, nc = lp / kVec16, na = rho ? 5 : 1;
+    const int tp = S.nt * lp;                       // points of a tile plane
+    const int npl = P.nz - 2 * R;
+    const int z = blockIdx.y, col = blockIdx.x;
+    const int k0 = R + col % gk * ty, j0 = R + col / gk * txr;
+    for (int t = threadIdx.x; t < tp; t += blockDim.x) {
+        const int x = t % kVec16, tid = t / kVec16 % S.nt, c = t / kVec16 / S.nt;
+        const int l = c * kVec16 + x, lane = tid % 64, lw = 64 / S.wr;
+        const int slot = tid / 64 * S.wr + lane / lw;
+        const int j = j0 + slot * S.rpt + l / S.v;
+        const int k = k0 + lane % lw * S.v + l % S.v;
+        const int i = R + z;
+        real_t v[5] = {0, 0, 0, 0, 0}, e = 0;
+        if (j < P.nx - R && k < P.ny - R) {
+            const long long p = (long long)i * P.sz + (long long)j * P.sx + k;
+            e = P.e[p];
+            v[0] = P.q[p] / (real_t)(1.0 + (double)e);
+            if (rho) {
+                const real_t *__restrict__ d = P.rho + p;
+                for (int m = 1; m <= R; m++) {
+                    v[1] += P.c1[m] * (d[m * P.sz] - d[-m * P.sz]);
+                    v[2] += P.c1[m] * (d[m * P.nx] - d[-m * P.nx]);
+                    v[3] += P.c1[m] * (d[m] - d[-m]);
+                }
+                v[4] = d[0];
+            }
+        }
+        const long long plane = (long long)col * npl + z;
+        for (int a = 0; a < na; a++)
+            pk[((plane * na + a) * nc + c) * (S.nt * kVec16) + tid * kVec16 + x] = v[a];
+        pe[(plane * nc + c) * (S.nt * kVec16) + tid * kVec16 + x] = e;
+    }
+}
+
 // Bits z0 .. z0+63 of a tile column's damping mask.
 __device__ __forceinline__ unsigned long long damp_bits(const Tiling &T, int col, int z0)
 {
@@ -248,8 +303,8 @@ __device__ __forceinline__ real_t leapfrog_plain(real_t value, real_t C, real_t 
 // The kernel's run constants, kept small so they stay in SGPRs.
 struct StepArgs {
     const real_t *uc, *up;
-    const real_t *qc;   // (dt2/s)/den per point
-    const real_t *e;
+    const real_t *pk;   // packed coefficients (k_pack_tiles)
+    const real_t *pe;   // packed damping terms
     real_t *un;
     int nz, nx, ny;
     unsigned pbytes;    // bytes per z plane (working type)
@@ -259,11 +314,21 @@ struct StepArgs {
     FixedDiv dvz, dvx, dvy;
     real_t div_lo, div_hi;  // numerator range safe for all three divisors
     double ry, rx, rz;      // RN(1/dy2) ... in float64 (quotient mode D64)
+    int d64_check;          // D64: subnormal quotients go through IEEE division
     real_t c2[kMaxR + 1];
+    // variable density: first-derivative coefficients and RN(1/(4 dy2)) ...
+    real_t c1[kMaxR + 1];
+    double r4y, r4x, r4z;
     int nsrc;
     const Box *sbox;
     Tiling T;
 };
+
+// Whether x is a subnormal number.
+__device__ __forceinline__ bool subnormal(float x)
+{
+    return __builtin_amdgcn_classf(x, 0x90);
+}
 
 template <int R, int WR, int RPT, int NW, int VP>
 struct TileShape {
@@ -279,16 +344,25 @@ struct TileShape {
     static constexpr int HX = (2 * R + SLOTS - 1) / SLOTS;
     static constexpr int NYV = TXR * 2 * HV;           // y-halo vectors per plane
     static constexpr int HY = (NYV + 64 * NW - 1) / (64 * NW);
+    static constexpr int LP = RPT * V;                 // points per lane
+    static constexpr int NC = LP / kVec16;             // 16-byte chunks per lane and value
+    static_assert(LP % kVec16 == 0, "a lane's packed values fill whole 16-byte chunks");
+    static constexpr int NA(int rho) { return rho ? 5 : 1; }   // packed values per point
 };
 
 // D64 (float32 only): the Laplacian quotients sum/h2 as RN(sum * RN(1/h2)),
-// the product in float64; equal to the IEEE float quotient for every float
-// sum when h2 = B 2^t (B odd) has t <= 0 and lies in [2^-126, 2^24), which
-// the host checks (the product is within 2^-52 of the quotient, every
-// non-float quotient at least 2^-49 from a rounding midpoint, and with t <= 0
-// no quotient in the subnormal range lands on a midpoint).  Otherwise the
+// the product in float64; equal to the IEEE float quotient wherever that is
+// normal or zero, for h2 in [2^-126, 2^24) (the product is within 2^-52 of
+// the quotient, every non-float quotient at least 2^-49 from a rounding
+// midpoint).  With h2 = B 2^t (B odd) and t <= 0 no quotient in the subnormal
+// range lands on a midpoint either; otherwise (d64_check) a wavefront with a
+// subnormal quotient takes IEEE divisions (a tie that rounds up out of the
+// subnormal range is the IEEE result, 2^-126 being even).  Otherwise the
 // fixed-divisor float quotients with their range vote.
-template <int R, int WR, int RPT, int NW, int VP, bool D64 = false>
+// RHO: 0 constant density; 1 variable density; 2 variable density with
+// nx != ny, where the x-axis first derivatives read other points than the x
+// neighbours.
+template <int R, int WR, int RPT, int NW, int VP, bool D64 = false, int RHO = 0>
 __global__ void __launch_bounds__(64 * NW)
 k_step3d_vec(StepArgs A, const Params *__restrict__ Pd, int n)
 {
@@ -297,8 +371,9 @@ k_step3d_vec(StepArgs A, const Params *__restrict__ Pd, int n)
     constexpr int V = S::V, LW = S::LW, TY = S::TY, TXR = S::TXR, PADL = S::PADL;
     constexpr int HV = S::HV, LS = S::LS, H = S::H, SLOTS = S::SLOTS, HX = S::HX;
     constexpr int NYV = S::NYV, HY = S::HY;
-    constexpr int NT = 64 * NW;
+    constexpr int NT = 64 * NW, NA = S::NA(RHO), LP = S::LP, NC = S::NC;
     constexpr unsigned esz = sizeof(real_t);
+    typedef typename LaneVec<kVec16>::type vec16;
     // two plane buffers, each followed by one dump slot per thread that
     // takes the halo writes of lanes without a halo vector, so that every
     // lane issues the same LDS stores (no branches around them)
@@ -337,9 +412,12 @@ k_step3d_vec(StepArgs A, const Params *__restrict__ Pd, int n)
     const unsigned long long rem = (unsigned long long)(z1 + R - zb) * PB;
     const rsrc_t r_uc = make_rsrc(A.uc + off0 / esz, rem);
     const rsrc_t r_up = make_rsrc(A.up + off0 / esz, rem);
-    const rsrc_t r_q = make_rsrc(A.qc + off0 / esz, rem);
-    const rsrc_t r_e = make_rsrc(A.e + off0 / esz, rem);
     const rsrc_t r_un = make_rsrc(A.un + off0 / esz, rem);
+    // the tile's packed planes z0 .. z1-1
+    constexpr unsigned PKB = NA * NT * LP * esz, PEB = NT * LP * esz;
+    const unsigned long long plane0 = (unsigned long long)col * (nz - 2 * R) + (z0 - R);
+    const rsrc_t r_pk = make_rsrc((const char *)A.pk + plane0 * PKB, (unsigned)(z1 - z0) * PKB);
+    const rsrc_t r_pe = make_rsrc((const char *)A.pe + plane0 * PEB, (unsigned)(z1 - z0) * PEB);
 
     // This lane's points: rows j0 + slot*RPT + q (adjacent rows share their
     // x neighbours), columns k .. k+V-1.
@@ -357,6 +435,8 @@ k_step3d_vec(StepArgs A, const Params *__restrict__ Pd, int n)
         cb[q] = ((unsigned)jl * (unsigned)ny + (unsigned)kl) * esz;
     }
     const bool full = k + V <= ny - R;      // every point of the vector is interior
+    // this lane's packed values; lanes with no interior point load nothing
+    const unsigned pk_off = act[0] && k < ny - R ? (unsigned)tid * 16u : kOOB;
     // x halo: rows j0-R .. j0-1 and j0+TXR .. j0+TXR+R-1
     unsigned xh_off[HX];
     int xh_lds[HX];
@@ -455,7 +535,13 @@ k_step3d_vec(StepArgs A, const Params *__restrict__ Pd, int n)
     // halos for plane i+1 are loaded right after plane i is written to LDS;
     // u_prev, C and the damping term for plane i+1 right after plane i's
     // update has consumed them.
-    vreal nc[RPT], np[RPT], nq[RPT], ne[RPT], nhx[HX], nhy[HY];
+    vreal nc[RPT], np[RPT], nhx[HX], nhy[HY];
+    // C (then, variable density, the density's z, x and y derivative sums
+    // and the density itself) and the damping term
+    vec16 npk[NA][NC], npe[NC];
+    auto packed = [&](const vec16 (&v)[NC], int q, int e) {
+        return v[(q * V + e) / kVec16][(q * V + e) % kVec16];
+    };
     const unsigned long long dbits = damp_bits(T, col, z0);
     const bool den_ok = T.dmask[(long long)T.ncols * T.nwords] == 0;
     auto load_centre = [&](int I) {
@@ -471,18 +557,26 @@ k_step3d_vec(StepArgs A, const Params *__restrict__ Pd, int n)
         for (int h = 0; h < HY; h++)
             nhy[h] = vload<V>(r_uc, yh_off[h], sp);
     };
+    auto load_packed = [&](int I, bool live, bool damp) {
+        const unsigned sk = live ? (unsigned)(I - z0) * PKB : 0u;
+        const unsigned se = live ? (unsigned)(I - z0) * PEB : 0u;
+#pragma unroll
+        for (int a = 0; a < NA; a++)
+#pragma unroll
+            for (int c = 0; c < NC; c++)
+                npk[a][c] = vload<kVec16>(r_pk, live ? pk_off : kOOB,
+                                          sk + (unsigned)(a * NC + c) * NT * 16);
+        if (CLEAN || damp)
+#pragma unroll
+            for (int c = 0; c < NC; c++)
+                npe[c] = vload<kVec16>(r_pe, damp ? pk_off : kOOB, se + (unsigned)c * NT * 16);
+    };
     auto load_update = [&](int I) {
         const unsigned sp = (unsigned)(I - zb) * PB;
 #pragma unroll
-        for (int q = 0; q < RPT; q++) {
+        for (int q = 0; q < RPT; q++)
             np[q] = vload<V>(r_up, cb[q], sp);
-            nq[q] = vload<V>(r_q, cb[q], sp);
-        }
-        if ((dbits >> (I - z0)) & 1) {
-#pragma unroll
-            for (int q = 0; q < RPT; q++)
-                ne[q] = vload<V>(r_e, cb[q], sp);
-        }
+        load_packed(I, true, (dbits >> (I - z0)) & 1);
     };
     // Clean-tile loads: always issued; the prefetch past the last plane
     // and the damping term of undamped planes read kOOB (no traffic).
@@ -502,14 +596,11 @@ k_step3d_vec(StepArgs A, const Params *__restrict__ Pd, int n)
     };
     auto load_update_clean = [&](int I) {
         const bool live = I < z1;
-        const bool damp = live && ((dbits >> (I - z0)) & 1);
         const unsigned sp = live ? (unsigned)(I - zb) * PB : 0u;
 #pragma unroll
-        for (int q = 0; q < RPT; q++) {
+        for (int q = 0; q < RPT; q++)
             np[q] = vload<V>(r_up, live ? cb[q] : kOOB, sp);
-            nq[q] = vload<V>(r_q, live ? cb[q] : kOOB, sp);
-            ne[q] = vload<V>(r_e, damp ? cb[q] : kOOB, sp);
-        }
+        load_packed(I, live, live && ((dbits >> (I - z0)) & 1));
     };
     // The scheduler barriers keep the prologue's loads in the loop's order
     // (centre and halos before the update operands), so the wait counts
@@ -560,6 +651,7 @@ k_step3d_vec(StepArgs A, const Params *__restrict__ Pd, int n)
         const bool special = !CLEAN && ((smask != 0) | bc_here);
         const unsigned so = (unsigned)(i - zb) * PB;
         vreal out[RPT];
+        vreal duz[RPT], dux[RPT], duy[RPT];   // variable density
         // x neighbours of the lane's RPT adjacent rows: rows -R .. RPT-1+R
         // around its first row, the own rows from registers
         // (one row per lane: read inside the stencil loop instead, which
@@ -614,14 +706,54 @@ k_step3d_vec(StepArgs A, const Params *__restrict__ Pd, int n)
                     acc_x[e] += A.c2[m] * (xp[e] + xm[e]);
                     acc_z[e] += A.c2[m] * (qz[q][R + m][e] + qz[q][R - m][e]);
                 }
+                if constexpr (RHO != 0) {
+                    // the reference steps along x by nx elements
+                    // (vd-3d wave.c:184-186): other points than x
+                    // neighbours unless nx == ny
+                    if constexpr (RHO == 2) {
+                        const unsigned o = (unsigned)(m * nx) * esz;
+                        xp = vload<V>(r_uc, cb[q] + so + o, 0u);
+                        xm = vload<V>(r_uc, cb[q] + so - o, 0u);
+                    }
+#pragma unroll
+                    for (int e = 0; e < V; e++) {
+                        const real_t dy = A.c1[m] * (win[PADL + e + m] - win[PADL + e - m]);
+                        const real_t dx = A.c1[m] * (xp[e] - xm[e]);
+                        const real_t dz = A.c1[m] * (qz[q][R + m][e] - qz[q][R - m][e]);
+                        // the sums start at +0 in the reference; whether a
+                        // sum is +0 or -0 reaches no stored bit
+                        duy[q][e] = m == 1 ? dy : duy[q][e] + dy;
+                        dux[q][e] = m == 1 ? dx : dux[q][e] + dx;
+                        duz[q][e] = m == 1 ? dz : duz[q][e] + dz;
+                    }
+                }
             }
             real_t lap[V];
             if constexpr (D64) {
+                float ly[V], lx[V], lz[V];
+#pragma unroll
+                for (int e = 0; e < V; e++) {
+                    ly[e] = (float)((double)acc_y[e] * A.ry);
+                    lx[e] = (float)((double)acc_x[e] * A.rx);
+                    lz[e] = (float)((double)acc_z[e] * A.rz);
+                }
+                if (A.d64_check) {
+                    bool sub = false;
+#pragma unroll
+                    for (int e = 0; e < V; e++)
+                        sub |= subnormal(ly[e]) | subnormal(lx[e]) | subnormal(lz[e]);
+                    if (__any(sub)) {
+#pragma unroll
+                        for (int e = 0; e < V; e++) {
+                            ly[e] = (float)acc_y[e] / (float)A.dy2;
+                            lx[e] = (float)acc_x[e] / (float)A.dx2;
+                            lz[e] = (float)acc_z[e] / (float)A.dz2;
+                        }
+                    }
+                }
 #pragma unroll
                 for (int e = 0; e < V; e++)
-                    lap[e] = (real_t)((double)acc_y[e] * A.ry) +
-                             (real_t)((double)acc_x[e] * A.rx) +
-                             (real_t)((double)acc_z[e] * A.rz);
+                    lap[e] = ly[e] + lx[e] + lz[e];
             } else {
             // Fixed-divisor quotients for every point; the IEEE quotients
             // replace them where a numerator is outside the safe range (or
@@ -661,12 +793,53 @@ k_step3d_vec(StepArgs A, const Params *__restrict__ Pd, int n)
         // branch per point, folded into the stencil, waited for them at the
         // start of the plane).
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (RHO != 0) {
+            // value -= (t_y + t_x + t_z) / rho, t = (du drho) / (4 h2)
+            // (vd-3d wave.c:199-204)
+#pragma unroll
+            for (int q = 0; q < RPT; q++) {
+                real_t ty[V], tx[V], tz[V];
+                if constexpr (D64) {
+#pragma unroll
+                    for (int e = 0; e < V; e++) {
+                        ty[e] = (real_t)((double)(duy[q][e] * packed(npk[3], q, e)) * A.r4y);
+                        tx[e] = (real_t)((double)(dux[q][e] * packed(npk[2], q, e)) * A.r4x);
+                        tz[e] = (real_t)((double)(duz[q][e] * packed(npk[1], q, e)) * A.r4z);
+                    }
+                    if (A.d64_check) {
+                        bool sub = false;
+#pragma unroll
+                        for (int e = 0; e < V; e++)
+                            sub |= subnormal(ty[e]) | subnormal(tx[e]) | subnormal(tz[e]);
+                        if (__any(sub)) {
+#pragma unroll
+                            for (int e = 0; e < V; e++) {
+                                ty[e] = (duy[q][e] * packed(npk[3], q, e)) / (4 * A.dy2);
+                                tx[e] = (dux[q][e] * packed(npk[2], q, e)) / (4 * A.dx2);
+                                tz[e] = (duz[q][e] * packed(npk[1], q, e)) / (4 * A.dz2);
+                            }
+                        }
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < V; e++) {
+                        ty[e] = (duy[q][e] * packed(npk[3], q, e)) / (4 * A.dy2);
+                        tx[e] = (dux[q][e] * packed(npk[2], q, e)) / (4 * A.dx2);
+                        tz[e] = (duz[q][e] * packed(npk[1], q, e)) / (4 * A.dz2);
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < V; e++)
+                    out[q][e] -= (ty[e] + tx[e] + tz[e]) / packed(npk[4], q, e);
+            }
+        }
         auto update = [&](auto f) {
 #pragma unroll
             for (int q = 0; q < RPT; q++)
 #pragma unroll
                 for (int e = 0; e < V; e++)
-                    out[q][e] = f(out[q][e], nq[q][e], ne[q][e], qz[q][R][e], np[q][e]);
+                    out[q][e] = f(out[q][e], packed(npk[0], q, e), packed(npe, q, e),
+                                  qz[q][R][e], np[q][e]);
         };
         if (!damped)
             update([](real_t v, real_t C, real_t, real_t uc, real_t up) {

@@ -237,11 +237,13 @@ class DeviceForward:
     @property
     def device_bytes(self):
         """HBM this shot holds while planned: slots, models, shot record and
-        the library's per-point arrays (q, damping term, (dt^2/s)/den and
-        the density copy)."""
+        the library's per-point arrays (q, damping term, their copies in tile
+        order and, with variable density, the density's derivative sums and
+        copy)."""
         total = sum(t.numel() * t.element_size() for t in self.tensors.values())
         vel = self.tensors["velocity_model"]
-        return total + 4 * vel.numel() * vel.element_size()
+        arrays = 8 if "density_model" in self.tensors else 4
+        return total + arrays * vel.numel() * vel.element_size()
 
     @property
     def steps(self):

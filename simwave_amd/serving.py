@@ -48,9 +48,9 @@ def percentile(values, q):
 
 def shot_bytes(solver):
     """HBM an admitted shot holds: wavefield slots, models, shot record and
-    the library's per-point arrays (q, damping term, (dt^2/s)/den, density
-    copy and, for variable density from space order 12, the density
-    derivative sums)."""
+    the library's per-point arrays (q, damping term and, in tile order and
+    padded to whole tiles, (dt^2/s)/den and the damping term; with variable
+    density the density's derivative sums and copy too)."""
     if hasattr(solver, "device_bytes"):           # test doubles
         return float(solver.device_bytes)
     sm = solver.space_model
@@ -58,9 +58,8 @@ def shot_bytes(solver):
     esz = np.dtype(sm.dtype).itemsize
     slots = solver.num_snapshots + 2
     models = 3 if sm.density_model is not None else 2
-    # variable density from space order 12: the density derivative sums
-    sums = len(sm.extended_shape) if (sm.density_model is not None
-                                       and sm.space_order >= 12) else 0
+    # variable density in 3D: derivative sums and the density in tile order
+    sums = len(sm.extended_shape) + 1 if sm.density_model is not None else 0
     rec = solver.time_model.timesteps * solver.receivers.count
     return float((slots + models + 4 + sums) * npts * esz + rec * esz)
 
