@@ -1,10 +1,10 @@
 // Batched step kernels for the shot server on gfx950.
 //
 // One launch advances several stride-0 shots of the same radius by one time
-// step each: the blocks of the launch are the shots' own step grids laid
-// end to end, and every block finds its shot by a search over the prefix
+// step each: the blocks of the launch are the shots' own receiver and step
+// grids laid end to end, and every block finds its shot by a search over the prefix
 // of block counts (kernel arguments), then runs the single-shot block body
-// (step3d_z_block / step2d_z_block / receivers_coop_block) on that shot's
+// (step3d_z_block / step2d_z_block / receivers_block) on that shot's
 // arrays with its step number.  Same operations per point as the
 // single-shot kernels, so a batched shot gives the same bits as it alone.
 // Slots follow the stride-0 cycle of the reference's time loop
@@ -25,12 +25,18 @@ struct BatchShot {
     const Box *rbox;
     const real_t *rw;
     long long npts;            // slot stride (points)
-    int nrec;
+    int nrec, nrb;             // receivers and their blocks, ahead of the step's
     int zlen;                  // z chunk of the step grid
     int gx, gy;                // step grid: blocks along the contiguous axis, then x
 };
 
 constexpr int kMaxBatch = 48;
+
+#if SW_DIM == 3
+constexpr int kBatchLines = kZLines, kRecPerBatch = kRecPerZ, kRecChunkBatch = kRecChunkZ;
+#else
+constexpr int kBatchLines = 4, kRecPerBatch = sizeof(real_t) == 4 ? 16 : 8, kRecChunkBatch = 128;
+#endif
 
 // Arguments of one batched launch (by value): the shots, their step numbers
 // and the first block of each (first[count] = blocks of the launch).
@@ -54,53 +60,42 @@ __device__ __forceinline__ int batch_shot(const BatchArgs &A, int b)
     return lo;
 }
 
-#if SW_DIM == 3
 template <int R>
+#if SW_DIM == 3
 __global__ void __launch_bounds__(64 * kZLines)
 k_step3d_z_batch(BatchArgs A)
-{
-    const int s = batch_shot(A, blockIdx.x);
-    const BatchShot *__restrict__ b = A.shot[s];
-    const Params P = b->P;
-    const LapDiv D = b->D;
-    const int n = A.n[s];
-    const int local = blockIdx.x - A.first[s];
-    const int gx = b->gx, gy = b->gy;
-    const int bx = local % gx, t = local / gx;
-    const long long np = b->npts;
-    real_t *u = b->u;
-    step3d_z_block<R>(P, D, u + (long long)(n % 3) * np, u + (long long)((n - 1) % 3) * np,
-                      u + (long long)((n + 1) % 3) * np, n, b->zlen, bx, t % gy, t / gy);
-}
 #else
-template <int R>
 __global__ void __launch_bounds__(kZ2Block)
 k_step2d_z_batch(BatchArgs A)
+#endif
 {
+    constexpr int NT = SW_DIM == 3 ? 64 * kBatchLines : 256;
+    __shared__ RecShared<kRecPerBatch, kRecChunkBatch> sh;
     const int s = batch_shot(A, blockIdx.x);
     const BatchShot *__restrict__ b = A.shot[s];
     const Params P = b->P;
     const int n = A.n[s];
-    const int local = blockIdx.x - A.first[s];
-    const int gx = b->gx;
+    int local = blockIdx.x - A.first[s];
     const long long np = b->npts;
     real_t *u = b->u;
-    step2d_z_block<R>(P, u + (long long)(n % 3) * np, u + (long long)((n - 1) % 3) * np,
-                      u + (long long)((n + 1) % 3) * np, n, b->zlen, local % gx, local / gx);
-}
+    const real_t *uc = u + (long long)(n % 3) * np;
+    if (local < b->nrb) {
+        receivers_block<NT>(P, sh, uc, b->rbox, b->rw, b->nrec,
+                            b->rec + (long long)(n - 1) * b->nrec, local,
+                            SW_DIM == 3 ? threadIdx.y * 64 + threadIdx.x : threadIdx.x);
+        return;
+    }
+    local -= b->nrb;
+    const int gx = b->gx;
+    const real_t *up = u + (long long)((n - 1) % 3) * np;
+    real_t *un = u + (long long)((n + 1) % 3) * np;
+#if SW_DIM == 3
+    const LapDiv D = b->D;
+    const int gy = b->gy, t = local / gx;
+    step3d_z_block<R>(P, D, uc, up, un, n, b->zlen, local % gx, t % gy, t / gy);
+#else
+    step2d_z_block<R>(P, uc, up, un, n, b->zlen, local % gx, local / gx);
 #endif
-
-template <int RPB, int CH>
-__global__ void __launch_bounds__(256)
-k_receivers_batch(BatchArgs A)
-{
-    const int s = batch_shot(A, blockIdx.x);
-    const BatchShot *__restrict__ b = A.shot[s];
-    const Params P = b->P;
-    const int n = A.n[s];
-    receivers_coop_block<RPB, CH>(P, b->u + (long long)(n % 3) * b->npts, b->rbox, b->rw,
-                                  b->nrec, b->rec + (long long)(n - 1) * b->nrec,
-                                  blockIdx.x - A.first[s]);
 }
 
 }  // namespace sw

@@ -379,8 +379,8 @@ struct Prepared {
     int zmarch_zlen = 16;
     sw::LapDiv lapdiv{};         // its fixed-divisor quotients
     bool tiled = false;          // use k_step3d_vec
-    void (*tiled_launch)(const struct Prepared &, const real_t *, const real_t *,
-                         real_t *, int, hipStream_t, LaunchTimer) = nullptr;
+    void (*tiled_launch)(const struct Prepared &, const real_t *, const real_t *, real_t *, int,
+                         hipStream_t, LaunchTimer, sw::RecArgs) = nullptr;
     const Params *Pd = nullptr;   // device copy of P for the tiled kernel
     const real_t *pk = nullptr, *pe = nullptr;   // its packed coefficients (k_pack_tiles)
     bool fastdiv = false;
@@ -846,7 +846,7 @@ bool prefer_tiled_vd(const Prepared &pr, bool oblong, const DeviceArena &arena)
 
 template <int R, int WR, int RPT, int NW, int V, bool D64, int RHO>
 void tiled_launch(const Prepared &pr, const real_t *uc, const real_t *up, real_t *un,
-                  int n, hipStream_t st, LaunchTimer tm)
+                  int n, hipStream_t st, LaunchTimer tm, sw::RecArgs rec)
 {
     const Params &P = pr.P;
     sw::StepArgs A{};
@@ -887,12 +887,21 @@ void tiled_launch(const Prepared &pr, const real_t *uc, const real_t *up, real_t
     A.nsrc = P.nsrc;
     A.sbox = P.sbox;
     A.T = pr.tiling;
-    launch_timed(sw::k_step3d_vec<R, WR, RPT, NW, V, D64, RHO>, dim3(pr.tiled_blocks), dim3(64, NW),
-                 st, tm, A, pr.Pd, n);
+    rec.nrb = (rec.nrec + sw::kRecPerWave * NW - 1) / (sw::kRecPerWave * NW);
+    rec.nrb = (rec.nrb + 7) / 8 * 8;
+    // the gather's blocks, in groups of 8, spread over the first three quarters
+    // of the launch: all at the front they delay the step (472^3: 57.6 ms per
+    // 100 steps, spread 55.6), spread to the end some finish after it (276^3
+    // variable density so8 21.1 ms, front 20.1, this 20.0)
+    const long long groups = ((long long)pr.tiled_blocks + rec.nrb + 7) / 8;
+    rec.period = rec.nrb ? (int)std::max(1ll, groups * 3 / 4 / (rec.nrb / 8)) : 1;
+    A.rec = rec;
+    launch_timed(sw::k_step3d_vec<R, WR, RPT, NW, V, D64, RHO>, dim3(pr.tiled_blocks + rec.nrb),
+                 dim3(64, NW), st, tm, A, pr.Pd, n);
 }
 
 using TiledFn = void (*)(const Prepared &, const real_t *, const real_t *, real_t *, int,
-                         hipStream_t, LaunchTimer);
+                         hipStream_t, LaunchTimer, sw::RecArgs);
 struct TiledKernel {
     TiledFn launch;
     TiledFn launch64;   // float64-reciprocal quotients (float32 builds)
@@ -1319,18 +1328,23 @@ struct RecStream {
 #if SW_DIM == 3
 // One step of k_step3d_z over the interior.
 void zmarch_launch(const Prepared &pr, const real_t *uc, const real_t *up, real_t *un, int n,
-                   hipStream_t st, LaunchTimer tm)
+                   hipStream_t st, LaunchTimer tm, sw::RecArgs rec)
 {
     const Params &P = pr.P;
     const int R = pr.r, zl = pr.zmarch_zlen;
-    const dim3 grid((unsigned)((P.ny - 2 * R + 63) / 64),
-                    (unsigned)((P.nx - 2 * R + sw::kZLines - 1) / sw::kZLines),
-                    (unsigned)((P.nz - 2 * R + zl - 1) / zl));
+    const int gx = (P.ny - 2 * R + 63) / 64;
+    const int gy = (P.nx - 2 * R + sw::kZLines - 1) / sw::kZLines;
+    const long long blocks = (long long)gx * gy * ((P.nz - 2 * R + zl - 1) / zl);
+    rec.nrb = (rec.nrec + sw::kRecPerZ - 1) / sw::kRecPerZ;
+    if (blocks + rec.nrb >= (1ll << 31))
+        fail("grid of %lld blocks is too large for one launch", blocks);
+    const dim3 grid((unsigned)(blocks + rec.nrb));
     const dim3 block(64, sw::kZLines);
     switch (R) {
 #define SW_Z_CASE(RR)                                                                   \
     case RR:                                                                            \
-        launch_timed(sw::k_step3d_z<RR>, grid, block, st, tm, P, pr.lapdiv, uc, up, un, n, zl); \
+        launch_timed(sw::k_step3d_z<RR>, grid, block, st, tm, P, pr.lapdiv, uc, up, un, n, zl, \
+                     gx, gy, rec);                                                      \
         return;
     SW_Z_CASE(1) SW_Z_CASE(2) SW_Z_CASE(3) SW_Z_CASE(4) SW_Z_CASE(5)
     SW_Z_CASE(6) SW_Z_CASE(7) SW_Z_CASE(8) SW_Z_CASE(9) SW_Z_CASE(10)
@@ -1347,11 +1361,13 @@ void zmarch_launch(const Prepared &pr, const real_t *uc, const real_t *up, real_
 // `swap` exchanges two logical slots.
 //
 // The receiver gather of step n only reads u^n (slot cur(n)), which no step
-// before n+2 writes in the reference's slot cycle, so it runs on a second
-// stream concurrently with the following kernels.  Ordering: it starts after
-// everything enqueued before step n on `st` (u^n complete); `st` waits for
-// it before any later step whose output slot is cur(n), before step n+2 in
-// any case, before uploads into recycled buffers and before slot exchanges.
+// before n+2 writes in the reference's slot cycle, so it rides in the step's
+// launch (z-marching and tiled kernels, RecArgs) or, for the other kernels
+// with kFlagOverlapReceivers, runs on a second stream beside the following
+// kernels.  Ordering there: it starts after everything enqueued before step
+// n on `st` (u^n complete); `st` waits for it before any later step whose
+// output slot is cur(n), before step n+2 in any case, before uploads into
+// recycled buffers and before slot exchanges.
 //
 // With kFlagTimeSteps every fused step kernel is launched with its own
 // event pair, set by the runtime at the kernel's start and end (the generic
@@ -1389,9 +1405,18 @@ void time_loop(const Args &a, const Prepared &pr, const std::vector<StepSlots> &
         for (hipEvent_t &e : tev.t)
             hip_check(hipEventCreate(&e), "hipEventCreate");
     }
-    // the overlap costs three extra stream operations per step: worth it
-    // where a step kernel is long enough to hide the gather
-    const bool overlap_rec = a.nrec && (flags & kFlagOverlapReceivers) &&
+    const bool coop_receivers = !env_flag("SIMWAVE_HIP_REC_THREAD");
+    // the z-marching and tiled steps carry their receiver gather (RecArgs)
+#if SW_DIM == 2
+    const bool carries = pr.fused && zmarch_2d(r);
+#else
+    const bool carries = pr.fused && (pr.zmarch || pr.tiled);
+#endif
+    const bool rec_in_step =
+        carries && a.nrec && coop_receivers && !env_flag("SIMWAVE_HIP_REC_SEPARATE");
+    // for the other kernels, on request and on large grids, a second stream:
+    // it costs three extra stream operations per step
+    const bool overlap_rec = a.nrec && !rec_in_step && (flags & kFlagOverlapReceivers) &&
                              pr.npts >= kOverlapMinPoints &&
                              !env_flag("SIMWAVE_HIP_REC_SERIAL");
     if (overlap_rec)
@@ -1406,14 +1431,6 @@ void time_loop(const Args &a, const Prepared &pr, const std::vector<StepSlots> &
         hip_check(hipStreamWaitEvent(st, ev.rec[j % 3], 0), "hipStreamWaitEvent");
     };
     const unsigned rec_blocks = (unsigned)((a.nrec + 255) / 256);
-    const bool coop_receivers = !env_flag("SIMWAVE_HIP_REC_THREAD");
-#if SW_DIM == 2
-    // 2D z-marching steps carry their receiver gather (one launch per step)
-    const bool rec_in_step = pr.fused && a.nrec && !overlap_rec && coop_receivers &&
-                             zmarch_2d(r) && !env_flag("SIMWAVE_HIP_REC_SEPARATE");
-#else
-    const bool rec_in_step = false;
-#endif
     const unsigned coop_blocks = (unsigned)((a.nrec + kRecPerBlock - 1) / kRecPerBlock);
     auto receivers = [&](size_t n, const real_t *uc, hipStream_t s) {
         real_t *row = rec_dev + (n - 1 - rec_row0) * a.nrec;
@@ -1454,10 +1471,14 @@ void time_loop(const Args &a, const Prepared &pr, const std::vector<StepSlots> &
                                    (int)n, 1);
             const LaunchTimer tm{t0, t1};
 #if SW_DIM == 3
+            sw::RecArgs rec{};
+            if (rec_in_step)
+                rec = sw::RecArgs{pr.rbox, pr.rw, rec_dev + (n - 1 - rec_row0) * a.nrec,
+                                  (int)a.nrec, 0, 1};
             if (pr.zmarch)
-                zmarch_launch(pr, uc, up, un, (int)n, st, tm);
+                zmarch_launch(pr, uc, up, un, (int)n, st, tm, rec);
             else if (pr.tiled)
-                pr.tiled_launch(pr, uc, up, un, (int)n, st, tm);
+                pr.tiled_launch(pr, uc, up, un, (int)n, st, tm, rec);
             else
 #else
             if (rec_in_step)
@@ -1978,10 +1999,10 @@ struct Plan {
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     // batched runs (run_plans_batched): the shot's constants on the device
-    // and the blocks of its step and receiver grids; null when the plan
-    // runs only on its own
+    // and the blocks of its receiver and step grids together; null when the
+    // plan runs only on its own
     const sw::BatchShot *bshot = nullptr;
-    int bblocks = 0, rblocks = 0;
+    int bblocks = 0;
     // whole-run 2D launches (k_step2d_persist): the barrier counter and the
     // abort word; null when the plan runs step by step
     unsigned *bar = nullptr;
@@ -2107,12 +2128,12 @@ void setup_batch(Plan &p)
     b.rw = pr.rw;
     b.npts = pr.npts;
     b.nrec = (int)p.a.nrec;
+    b.nrb = (b.nrec + sw::kRecPerBatch - 1) / sw::kRecPerBatch;
     sw::BatchShot *d = p.arena.alloc<sw::BatchShot>(1);
     hip_check(hipMemcpyAsync(d, &b, sizeof(b), hipMemcpyHostToDevice, p.st),
               "copy batch constants");
     p.bshot = d;
-    p.bblocks = (int)blocks;
-    p.rblocks = (int)((p.a.nrec + kRecPerBlock - 1) / kRecPerBlock);
+    p.bblocks = (int)blocks + b.nrb;
 }
 
 template <int R>
@@ -2137,9 +2158,8 @@ constexpr BatchFn kStepBatch[] = {nullptr,
 
 // Enqueues up to `steps` further steps of every plan on `st`, after each
 // plan's earlier work.  Plans that can be batched (setup_batch) advance
-// together, radius by radius, up to kMaxBatch per launch: one step kernel
-// and one receiver kernel per time step for all of them, in segments over
-// which the set of unfinished plans is fixed.  The others run on their own
+// together, radius by radius, up to kMaxBatch per launch: one kernel per time
+// step takes the steps and receivers of all of them, in segments over which the set of unfinished plans is fixed.  The others run on their own
 // (run_plan).  left[i]: steps plan i has left.
 void run_plans_batched(Plan *const *plans, int count, size_t steps, hipStream_t st,
                        long long *left)
@@ -2178,33 +2198,20 @@ void run_plans_batched(Plan *const *plans, int count, size_t steps, hipStream_t 
                 break;
             for (size_t c0 = 0; c0 < act.size(); c0 += sw::kMaxBatch) {
                 const int cnt = (int)std::min<size_t>(sw::kMaxBatch, act.size() - c0);
-                sw::BatchArgs S{}, Rc{};
+                sw::BatchArgs S{};
                 S.count = cnt;
                 S.first[0] = 0;
-                int rc = 0;
                 for (int i = 0; i < cnt; i++) {
                     const Plan *p = act[c0 + i];
                     S.shot[i] = p->bshot;
                     S.n[i] = (int)(p->a.n0 + p->done);
                     S.first[i + 1] = S.first[i] + p->bblocks;
-                    if (p->rblocks) {
-                        Rc.shot[rc] = p->bshot;
-                        Rc.n[rc] = S.n[i];
-                        Rc.first[rc + 1] = Rc.first[rc] + p->rblocks;
-                        rc++;
-                    }
                 }
-                Rc.count = rc;
                 for (size_t k = 0; k < seg; k++) {
                     kStepBatch[R](S, st);
-                    if (rc)
-                        hipLaunchKernelGGL((sw::k_receivers_batch<kRecPerBlock, kRecChunk>),
-                                           dim3((unsigned)Rc.first[rc]), dim3(256), 0, st, Rc);
                     hip_check(hipGetLastError(), "batched step");
                     for (int i = 0; i < cnt; i++)
                         S.n[i]++;
-                    for (int i = 0; i < rc; i++)
-                        Rc.n[i]++;
                 }
             }
             for (Plan *p : act)

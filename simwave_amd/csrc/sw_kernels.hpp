@@ -372,6 +372,167 @@ __device__ __forceinline__ void store_with_bc(const Params &P, real_t *un,
     }
 }
 
+// ------------------------------------------------ receivers
+// Receivers, cooperative form: a block of NT threads serves RPB receivers.
+// The NT/RPB consecutive threads of one receiver gather its box values and multiply
+// them by their weights into LDS (CH points per receiver per round), then
+// lane q of the first wave adds receiver q's products in box order.  Every
+// product and every partial sum is rounded exactly as in the reference's
+// sequential loop (wave.c:533-565); only the loads and multiplies run in
+// parallel.  What bounds it is latency: a block's loads and then its one
+// chain of dependent adds.  So a thread has NB box values in flight at a
+// time (their box positions follow by adding the thread stride's digits, no
+// division), the axis weights come from LDS, and the chain reads its
+// products 16 at a time by 16-byte LDS loads, one group ahead of the adds;
+// rows are padded with zeros up to whole groups, which changes no bit (the
+// sum starts at +0, so it is never -0).  LDS rows start 16 banks apart: the
+// writes of a wave's receivers do not collide.  16384 receivers of 9^3
+// points at 472^3: 28 us alone per step, 56 before (single loads, the
+// chain waiting for every LDS read).
+constexpr int kRecWeights = 64;           // weights kept in LDS per receiver
+
+template <int RPB, int CH>
+struct RecShared {
+    static constexpr int ROW = CH + 64 / (int)sizeof(real_t);
+    static_assert(CH * sizeof(real_t) % 256 == 0, "LDS row layout");
+    alignas(16) real_t prod[RPB][ROW];
+    real_t wts[RPB][kRecWeights + 1];
+    int counts[RPB], nweights[RPB];
+};
+
+// Receivers bx*RPB .. bx*RPB+RPB-1 of one shot; tid: the thread in the block.
+template <int NT, int RPB, int CH>
+__device__ __forceinline__ void receivers_block(const Params &P, RecShared<RPB, CH> &sh,
+                                                const real_t *__restrict__ uc,
+                                                const Box *__restrict__ rbox,
+                                                const real_t *__restrict__ rw, int nrec,
+                                                real_t *__restrict__ out, int bx, int tid)
+{
+    constexpr int STEP = NT / RPB;        // threads of one receiver
+    constexpr int NB = 8;                 // box values in flight per thread
+    constexpr int GRP = 16;               // products per step of the chain
+    constexpr int WCAP = kRecWeights;
+    static_assert(CH % GRP == 0 && RPB <= 64 && NT % RPB == 0, "block layout");
+    typedef real_t vec16 __attribute__((ext_vector_type(16 / sizeof(real_t))));
+    constexpr int V = 16 / (int)sizeof(real_t);
+    const int r0 = bx * RPB;
+    const int l = tid / STEP, s = tid % STEP;   // receiver served, thread in it
+    Box b{};
+    int cnt = 0, nw = 0;
+    if (r0 + l < nrec)
+        b = rbox[r0 + l];
+    const int cz = b.hi[0] - b.lo[0] + 1, cx = b.hi[1] - b.lo[1] + 1;
+#if SW_DIM == 3
+    const int cy = b.hi[2] - b.lo[2] + 1;
+#else
+    const int cy = 1;
+#endif
+    if (r0 + l < nrec) {
+        cnt = cz * cx * cy;
+        nw = cz + cx + (SW_DIM == 3 ? cy : 0);
+    }
+    if (s == 0) {
+        sh.counts[l] = cnt;
+        sh.nweights[l] = nw;
+    }
+    if (nw <= WCAP)
+        for (int i = s; i < nw; i += STEP)
+            sh.wts[l][i] = rw[b.woff + i];
+    __syncthreads();
+    int total_max = 0, nw_max = 0;
+#pragma unroll
+    for (int q = 0; q < RPB; q++) {
+        total_max = max(total_max, sh.counts[q]);
+        nw_max = max(nw_max, sh.nweights[q]);
+    }
+#if SW_DIM == 3
+    const long long p0 = (long long)b.lo[0] * P.sz + (long long)b.lo[1] * P.sx + b.lo[2];
+#else
+    const long long p0 = (long long)b.lo[0] * P.sz + b.lo[1];
+#endif
+    // the thread stride as box digits (z, x, y)
+    const int dk = STEP % cy, dj = STEP / cy % cx, di = STEP / cy / cx;
+    real_t acc = 0;
+    for (int base = 0; base < total_max; base += CH) {
+        const int n16 = (min(CH, total_max - base) + GRP - 1) / GRP * GRP;
+        // products base .. base+n16-1 of every receiver, zeros past its box;
+        // a thread past the end of its box stays at its last valid position
+        auto gather = [&](auto weight) {
+            int t = base + s;
+            int ii = 0, jj = 0, kk = 0;
+            if (t < cnt) {
+                ii = t / (cx * cy);
+                const int rem = t - ii * cx * cy;
+                jj = rem / cy;
+                kk = rem - jj * cy;
+            }
+            for (int c0 = s; c0 < n16; c0 += STEP * NB) {
+                real_t uv[NB], kv[NB];
+#pragma unroll
+                for (int m = 0; m < NB; m++) {
+#if SW_DIM == 3
+                    uv[m] = uc[p0 + (long long)ii * P.sz + (long long)jj * P.sx + kk];
+                    kv[m] = weight(ii) * weight(cz + jj) * weight(cz + cx + kk);
+#else
+                    uv[m] = uc[p0 + (long long)ii * P.sz + jj];
+                    kv[m] = weight(ii) * weight(cz + jj);
+#endif
+                    if (t + (m + 1) * STEP < cnt) {
+                        kk += dk;
+                        jj += dj;
+                        ii += di;
+                        if (kk >= cy) {
+                            kk -= cy;
+                            jj++;
+                        }
+                        if (jj >= cx) {
+                            jj -= cx;
+                            ii++;
+                        }
+                    }
+                }
+#pragma unroll
+                for (int m = 0; m < NB; m++) {
+                    const int c = c0 + m * STEP;
+                    if (c < n16)
+                        sh.prod[l][c] = t + m * STEP < cnt ? uv[m] * kv[m] : (real_t)0;
+                }
+                t += STEP * NB;
+            }
+        };
+        if (nw_max <= WCAP)
+            gather([&](int i) { return sh.wts[l][i]; });
+        else
+            gather([&](int i) { return rw[b.woff + i]; });
+        __syncthreads();
+        if (tid < RPB) {
+            const vec16 *row = (const vec16 *)&sh.prod[tid][0];
+            vec16 a[GRP / V];
+#pragma unroll
+            for (int m = 0; m < GRP / V; m++)
+                a[m] = row[m];
+            for (int c = 0; c < n16; c += GRP) {
+                vec16 nx[GRP / V];
+                const int cn = (c + GRP < n16 ? c + GRP : c) / V;
+#pragma unroll
+                for (int m = 0; m < GRP / V; m++)
+                    nx[m] = row[cn + m];
+#pragma unroll
+                for (int m = 0; m < GRP / V; m++)
+#pragma unroll
+                    for (int e = 0; e < V; e++)
+                        acc += a[m][e];
+#pragma unroll
+                for (int m = 0; m < GRP / V; m++)
+                    a[m] = nx[m];
+            }
+        }
+        __syncthreads();
+    }
+    if (tid < RPB && r0 + tid < nrec)
+        out[r0 + tid] = acc;
+}
+
 // ------------------------------------------------ fused step, 3D
 // One workgroup = TY (=64, one wavefront row) points along the contiguous
 // axis y x TX rows along x, marching along z over [z0, z0+zlen).  The
@@ -670,12 +831,41 @@ __device__ __forceinline__ void step3d_z_block(const Params &P, const LapDiv &D,
     }
 }
 
+// The receiver gather that rides in a step launch: blocks 0 .. nrb-1 gather
+// the receivers of level n, which the step reads and does not write; the
+// step's blocks follow (the tiled kernel spreads the gather's).  Beside the
+// step on a second stream the gather waited for free CUs until the step's last
+// wave, and the event waits between the streams left gaps of up to 20 us per
+// step (100 steps: 276^3 variable density so8 with 4096 receivers 21.0 -> 20.0
+// ms, 472^3 so8 with 16384 56.4 -> 55.6).
+struct RecArgs {
+    const Box *rbox;
+    const real_t *rw;
+    real_t *out;        // row of this step
+    int nrec, nrb;
+    int period;         // tiled kernel: every period-th group of 8 blocks gathers
+};
+
+// The z-marching kernels' gather: 16 receivers per block, rounds of 256 (128
+// in float64) products, 17 KB of LDS, which leaves the step's occupancy.
+constexpr int kRecPerZ = 16;
+constexpr int kRecChunkZ = sizeof(real_t) == 4 ? 256 : 128;
+
 template <int R>
 __global__ void __launch_bounds__(64 * kZLines)
 k_step3d_z(Params P, LapDiv D, const real_t *__restrict__ uc, const real_t *__restrict__ up,
-           real_t *__restrict__ un, int n, int zlen)
+           real_t *__restrict__ un, int n, int zlen, int gx, int gy, RecArgs rec)
 {
-    step3d_z_block<R>(P, D, uc, up, un, n, zlen, blockIdx.x, blockIdx.y, blockIdx.z);
+    __shared__ RecShared<kRecPerZ, kRecChunkZ> sh;
+    if ((int)blockIdx.x < rec.nrb) {
+        if (P.nbase)
+            rec.out += (long long)(*P.nbase) * rec.nrec;
+        receivers_block<64 * kZLines>(P, sh, uc, rec.rbox, rec.rw, rec.nrec, rec.out, blockIdx.x,
+                                      threadIdx.y * 64 + threadIdx.x);
+        return;
+    }
+    const int s = blockIdx.x - rec.nrb, t = s / gx;
+    step3d_z_block<R>(P, D, uc, up, un, n, zlen, s % gx, t % gy, t / gy);
 }
 #endif
 
@@ -1157,168 +1347,15 @@ k_receivers(Params P, const real_t *__restrict__ uc, const Box *__restrict__ rbo
     out[q] = acc;
 }
 
-// Receivers, cooperative form: a block serves RPB receivers.  The 256/RPB
-// consecutive threads of one receiver gather its box values and multiply
-// them by their weights into LDS (CH points per receiver per round), then
-// lane q of the first wave adds receiver q's products in box order.  Every
-// product and every partial sum is rounded exactly as in the reference's
-// sequential loop (wave.c:533-565); only the loads and multiplies run in
-// parallel.  What bounds it is latency: a block's loads and then its one
-// chain of dependent adds.  So a thread has NB box values in flight at a
-// time (their box positions follow by adding the thread stride's digits, no
-// division), the axis weights come from LDS, and the chain reads its
-// products 16 at a time by 16-byte LDS loads, one group ahead of the adds;
-// rows are padded with zeros up to whole groups, which changes no bit (the
-// sum starts at +0, so it is never -0).  LDS rows start 16 banks apart: the
-// writes of a wave's receivers do not collide.  16384 receivers of 9^3
-// points at 472^3: 28 us alone per step, 56 before (single loads, the
-// chain waiting for every LDS read).
-// Receivers bx*RPB .. bx*RPB+RPB-1 of one shot.
-template <int RPB, int CH>
-__device__ __forceinline__ void receivers_coop_block(const Params &P,
-                                                     const real_t *__restrict__ uc,
-                                                     const Box *__restrict__ rbox,
-                                                     const real_t *__restrict__ rw, int nrec,
-                                                     real_t *__restrict__ out, int bx)
-{
-    constexpr int STEP = 256 / RPB;       // threads of one receiver
-    constexpr int NB = 8;                 // box values in flight per thread
-    constexpr int GRP = 16;               // products per step of the chain
-    constexpr int ROW = CH + 64 / (int)sizeof(real_t);
-    constexpr int WCAP = 64;              // weights kept in LDS per receiver
-    static_assert(CH * sizeof(real_t) % 256 == 0 && CH % GRP == 0, "LDS row layout");
-    typedef real_t vec16 __attribute__((ext_vector_type(16 / sizeof(real_t))));
-    constexpr int V = 16 / (int)sizeof(real_t);
-    __shared__ __align__(16) real_t prod[RPB][ROW];
-    __shared__ real_t wts[RPB][WCAP + 1];
-    __shared__ int counts[RPB], nweights[RPB];
-    const int tid = threadIdx.x;
-    const int r0 = bx * RPB;
-    const int l = tid / STEP, s = tid % STEP;   // receiver served, thread in it
-    Box b{};
-    int cnt = 0, nw = 0;
-    if (r0 + l < nrec)
-        b = rbox[r0 + l];
-    const int cz = b.hi[0] - b.lo[0] + 1, cx = b.hi[1] - b.lo[1] + 1;
-#if SW_DIM == 3
-    const int cy = b.hi[2] - b.lo[2] + 1;
-#else
-    const int cy = 1;
-#endif
-    if (r0 + l < nrec) {
-        cnt = cz * cx * cy;
-        nw = cz + cx + (SW_DIM == 3 ? cy : 0);
-    }
-    if (s == 0) {
-        counts[l] = cnt;
-        nweights[l] = nw;
-    }
-    if (nw <= WCAP)
-        for (int i = s; i < nw; i += STEP)
-            wts[l][i] = rw[b.woff + i];
-    __syncthreads();
-    int total_max = 0, nw_max = 0;
-#pragma unroll
-    for (int q = 0; q < RPB; q++) {
-        total_max = max(total_max, counts[q]);
-        nw_max = max(nw_max, nweights[q]);
-    }
-#if SW_DIM == 3
-    const long long p0 = (long long)b.lo[0] * P.sz + (long long)b.lo[1] * P.sx + b.lo[2];
-#else
-    const long long p0 = (long long)b.lo[0] * P.sz + b.lo[1];
-#endif
-    // the thread stride as box digits (z, x, y)
-    const int dk = STEP % cy, dj = STEP / cy % cx, di = STEP / cy / cx;
-    real_t acc = 0;
-    for (int base = 0; base < total_max; base += CH) {
-        const int n16 = (min(CH, total_max - base) + GRP - 1) / GRP * GRP;
-        // products base .. base+n16-1 of every receiver, zeros past its box;
-        // a thread past the end of its box stays at its last valid position
-        auto gather = [&](auto weight) {
-            int t = base + s;
-            int ii = 0, jj = 0, kk = 0;
-            if (t < cnt) {
-                ii = t / (cx * cy);
-                const int rem = t - ii * cx * cy;
-                jj = rem / cy;
-                kk = rem - jj * cy;
-            }
-            for (int c0 = s; c0 < n16; c0 += STEP * NB) {
-                real_t uv[NB], kv[NB];
-#pragma unroll
-                for (int m = 0; m < NB; m++) {
-#if SW_DIM == 3
-                    uv[m] = uc[p0 + (long long)ii * P.sz + (long long)jj * P.sx + kk];
-                    kv[m] = weight(ii) * weight(cz + jj) * weight(cz + cx + kk);
-#else
-                    uv[m] = uc[p0 + (long long)ii * P.sz + jj];
-                    kv[m] = weight(ii) * weight(cz + jj);
-#endif
-                    if (t + (m + 1) * STEP < cnt) {
-                        kk += dk;
-                        jj += dj;
-                        ii += di;
-                        if (kk >= cy) {
-                            kk -= cy;
-                            jj++;
-                        }
-                        if (jj >= cx) {
-                            jj -= cx;
-                            ii++;
-                        }
-                    }
-                }
-#pragma unroll
-                for (int m = 0; m < NB; m++) {
-                    const int c = c0 + m * STEP;
-                    if (c < n16)
-                        prod[l][c] = t + m * STEP < cnt ? uv[m] * kv[m] : (real_t)0;
-                }
-                t += STEP * NB;
-            }
-        };
-        if (nw_max <= WCAP)
-            gather([&](int i) { return wts[l][i]; });
-        else
-            gather([&](int i) { return rw[b.woff + i]; });
-        __syncthreads();
-        if (tid < RPB) {
-            const vec16 *row = (const vec16 *)&prod[tid][0];
-            vec16 a[GRP / V];
-#pragma unroll
-            for (int m = 0; m < GRP / V; m++)
-                a[m] = row[m];
-            for (int c = 0; c < n16; c += GRP) {
-                vec16 nx[GRP / V];
-                const int cn = (c + GRP < n16 ? c + GRP : c) / V;
-#pragma unroll
-                for (int m = 0; m < GRP / V; m++)
-                    nx[m] = row[cn + m];
-#pragma unroll
-                for (int m = 0; m < GRP / V; m++)
-#pragma unroll
-                    for (int e = 0; e < V; e++)
-                        acc += a[m][e];
-#pragma unroll
-                for (int m = 0; m < GRP / V; m++)
-                    a[m] = nx[m];
-            }
-        }
-        __syncthreads();
-    }
-    if (tid < RPB && r0 + tid < nrec)
-        out[r0 + tid] = acc;
-}
-
 template <int RPB, int CH>
 __global__ void __launch_bounds__(256)
 k_receivers_coop(Params P, const real_t *__restrict__ uc, const Box *__restrict__ rbox,
                  const real_t *__restrict__ rw, int nrec, real_t *__restrict__ out)
 {
+    __shared__ RecShared<RPB, CH> sh;
     if (P.nbase)
         out += (long long)(*P.nbase) * nrec;
-    receivers_coop_block<RPB, CH>(P, uc, rbox, rw, nrec, out, blockIdx.x);
+    receivers_block<256>(P, sh, uc, rbox, rw, nrec, out, blockIdx.x, threadIdx.x);
 }
 
 #if SW_DIM == 2
@@ -1337,11 +1374,12 @@ k_step2d_z_rec(Params P, const real_t *__restrict__ uc, const real_t *__restrict
                real_t *__restrict__ out)
 {
     static_assert(kZ2Block == 256, "the gather's block shape");
+    __shared__ RecShared<RPB, CH> sh;
     const int b = blockIdx.x;
     if (b < nrb) {
         if (P.nbase)
             out += (long long)(*P.nbase) * nrec;
-        receivers_coop_block<RPB, CH>(P, uc, rbox, rw, nrec, out, b);
+        receivers_block<256>(P, sh, uc, rbox, rw, nrec, out, b, threadIdx.x);
         return;
     }
     const int s = b - nrb;
@@ -1404,6 +1442,7 @@ k_step2d_persist(Params P, real_t *__restrict__ u, long long np, int n0, int n1,
                  unsigned *count, int *abort, int spin_limit, int roll_spin, int roll_extra)
 {
     static_assert(kZ2Block == 256, "the gather's block shape");
+    __shared__ RecShared<RPB, CH> sh;
     // roll_extra > 0 (tests of the fallback) asks for arrivals that never come
     if (!grid_sync(count, gridDim.x + roll_extra, abort, roll_spin, 1))
         return;
@@ -1414,7 +1453,7 @@ k_step2d_persist(Params P, real_t *__restrict__ u, long long np, int n0, int n1,
         real_t *row = rec0 + (long long)(n - n0) * nrec;
         for (int b = blockIdx.x; b < nrb + nsb; b += gridDim.x) {
             if (b < nrb) {
-                receivers_coop_block<RPB, CH>(P, uc, rbox, rw, nrec, row, b);
+                receivers_block<256>(P, sh, uc, rbox, rw, nrec, row, b, threadIdx.x);
             } else {
                 const int s = b - nrb;
                 step2d_z_block<R>(P, uc, up, un, n, zlen, s % gx, s / gx);

@@ -321,8 +321,19 @@ struct StepArgs {
     double r4y, r4x, r4z;
     int nsrc;
     const Box *sbox;
+    RecArgs rec;        // nrb a multiple of 8: the step's blocks keep their XCDs
     Tiling T;
 };
+
+// Receivers per wavefront of the gather in the step launch, and products per
+// round (9 KB of LDS, no more than the step's tile).  A gathering wavefront
+// takes a step wavefront's registers, so it serves several receivers (100
+// steps of 472^3 with 16384 receivers: 59.1 ms at 2 per wavefront, 58.2 at 4,
+// 57.6 at 8).
+constexpr int kRecPerWave = 8;
+constexpr int kRecChunkVec = sizeof(real_t) == 4 ? 256 : 128;
+template <int NW>
+using RecVec = RecShared<kRecPerWave * NW, kRecChunkVec>;
 
 // Whether x is a subnormal number.
 __device__ __forceinline__ bool subnormal(float x)
@@ -377,27 +388,42 @@ k_step3d_vec(StepArgs A, const Params *__restrict__ Pd, int n)
     // two plane buffers, each followed by one dump slot per thread that
     // takes the halo writes of lanes without a halo vector, so that every
     // lane issues the same LDS stores (no branches around them)
-    constexpr int DUMP = H * LS;
-    __shared__ __align__(16) real_t lds[2][H * LS + NT * V];
+    constexpr int DUMP = H * LS, PLANE = H * LS + NT * V;
+    constexpr size_t lds_step = 2 * PLANE * esz, lds_rec = sizeof(RecVec<NW>);
+    __shared__ __align__(16) unsigned char smem[lds_step > lds_rec ? lds_step : lds_rec];
+    real_t *const lds = (real_t *)smem;
 
     const int lane = threadIdx.x, w = threadIdx.y;
     const int tid = w * 64 + lane;
     const int slot = w * WR + lane / LW;     // row slot of this lane
     const int lc = lane % LW;                // vector column of this lane
+    int bid = blockIdx.x;
+    if (A.rec.nrb) {
+        const int g = bid >> 3, ng = A.rec.nrb >> 3, rg = g / A.rec.period;
+        if (rg < ng && g == rg * A.rec.period) {
+            real_t *out = A.rec.out;
+            if (Pd->nbase)
+                out += (long long)(*Pd->nbase) * A.rec.nrec;
+            receivers_block<NT>(*Pd, *(RecVec<NW> *)smem, A.uc, A.rec.rbox, A.rec.rw,
+                                     A.rec.nrec, out, rg * 8 + (bid & 7), tid);
+            return;
+        }
+        bid -= 8 * min(ng, rg + 1);
+    }
     const int nx = A.nx, ny = A.ny, nz = A.nz;
     const unsigned PB = A.pbytes;
     const Tiling &T = A.T;
 
     int col, zc;
     if (T.order == 1) {
-        const int xcd = blockIdx.x & 7, s = blockIdx.x >> 3;
+        const int xcd = bid & 7, s = bid >> 3;
         zc = s / T.chunk;
         col = xcd * T.chunk + s % T.chunk;
         if (col >= T.ncols)
             return;
     } else {
-        col = blockIdx.x % T.ncols;
-        zc = blockIdx.x / T.ncols;
+        col = bid % T.ncols;
+        zc = bid / T.ncols;
     }
     const int kt = col % T.gk, jt = col / T.gk;
     const int k0 = R + kt * TY, j0 = R + jt * TXR;
@@ -623,7 +649,7 @@ k_step3d_vec(StepArgs A, const Params *__restrict__ Pd, int n)
     for (int q = 0; q < RPT; q++)
         st_off[q] = (act[q] && full) ? cb[q] : kOOB;
     for (int i = z0; i < z1; i++) {
-        real_t *lb = &lds[(i - z0) & 1][0];
+        real_t *lb = lds + ((i - z0) & 1) * PLANE;
         const bool damped = (dbits >> (i - z0)) & 1;
 #pragma unroll
         for (int q = 0; q < RPT; q++) {
