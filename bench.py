@@ -375,10 +375,10 @@ def run_fwi(args):
     forward, residual and reverse sweep with checkpoints every 20 steps.
     value = the 16 shots' forward updates / iteration seconds.  Outside the
     timed region the same gradient in float64 gives the float32 error.  The
-    roofline is the reverse update kernel's (k_adj_update_z, 13 grid
-    accesses per extended point: W, lambda^{n+1}, e, v, lambda^n, three
-    forward levels and the gradient sum read; lambda^n, lambda^{n+1},
-    lambda^{n-1} and the gradient sum written)."""
+    roofline is the reverse update kernel's (k_adj_update_tiled, on average
+    9.5 grid accesses per interior point: lambda^k, lambda^{k+1}, W, c read,
+    lambda^{k-1} and its W written; every other step four forward levels, v
+    and the gradient sum read, the sum written)."""
     import torch
     from simwave_amd import fwi, workloads
 
@@ -423,13 +423,16 @@ def run_fwi(args):
     roof = None
     if stats.get("update_launches"):
         avg = stats["update_s"] / stats["update_launches"]
-        npts = int(np.prod(kw["velocity_model"].shape))
-        nbytes = 13 * np.dtype(dtype).itemsize * npts
+        halo = kw["space_order"]
+        npts = int(np.prod([n - halo for n in kw["velocity_model"].shape]))
+        # per interior point: two adjoint levels, W and c in, a level and W
+        # out; for two steps at once four forward levels, v, the sums in and out
+        nbytes = int(9.5 * np.dtype(dtype).itemsize * npts)
         achieved = nbytes / avg / 1e9
         roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                "traffic": read_traffic("k_adj_update_z", args.workload, dtype),
-                "kernel": "k_adj_update_z", "avg_launch_us": round(avg * 1e6, 2),
+                "traffic": read_traffic("k_adj_update_tiled", args.workload, dtype),
+                "kernel": "k_adj_update_tiled", "avg_launch_us": round(avg * 1e6, 2),
                 "launches": int(stats["update_launches"]),
                 "algorithmic_bytes_per_launch": int(nbytes)}
         log("reverse update: %d launches, avg %.1f us, %.1f GB/s algorithmic"

@@ -2484,57 +2484,135 @@ double run_device_noalloc(const Args &a, hipStream_t st, unsigned flags)
 }
 
 // ------------------------------------------------------------- adjoint
-// Reverse interior update of one step: the z-marching kernels (3D, 2D);
-// the whole-grid k_adj_update for radii they do not carry.
-#if SW_DIM == 3
-template <int R>
-void adj_update_z(const sw::Params &P, hipStream_t st, LaunchTimer tm, const real_t *vel,
-                  real_t *ub, const real_t *W, real_t *ub1, real_t *ub2, const real_t *u0,
-                  const real_t *u1, const real_t *u2, real_t *gacc, int image)
+#if SW_DIM == 2 && !SW_VD
+// Rows per block of the 2D reverse update: about 512 blocks (480 x 980 so8:
+// 8.0 us, 9.0 with 256 blocks, 8.2 with 2048; 540 x 740 so12 in float64 11.0,
+// 12.1 with 2048; 940 x 1840 so8 17.2 and 16.5).
+int adj_zlen_2d(const Params &P, int R)
 {
-    const dim3 grid((unsigned)((P.ny + 63) / 64),
-                    (unsigned)((P.nx + sw::kAdjLines - 1) / sw::kAdjLines),
-                    (unsigned)((P.nz + sw::kAdjZChunk - 1) / sw::kAdjZChunk));
-    launch_timed(sw::k_adj_update_z<R>, grid, sw::adj_block(), st, tm, P, vel, ub, W, ub1, ub2,
-                 u0, u1, u2, gacc, image);
+    const int gx = (P.nx - 2 * R + 255) / 256, Iz = P.nz - 2 * R;
+    const int target = 512;
+    const int nzc = std::min(std::max(1, (target + gx - 1) / gx), Iz);
+    return (Iz + nzc - 1) / nzc;
 }
 #endif
 
-void adj_update(const sw::Params &P, hipStream_t st, LaunchTimer tm, const real_t *vel,
-                real_t *ub, const real_t *W, real_t *ub1, real_t *ub2, const real_t *u0,
-                const real_t *u1, const real_t *u2, real_t *gacc, int image)
+#if !SW_VD
+// Launch shape of the reverse updates of one gradient.
+struct AdjPlan {
+    unsigned halo_lines = 0;    // lines of the Neumann faces, in face order
+#if SW_DIM == 3
+    bool tiled = false;
+    sw::Tiling T{};
+    int tiled_blocks = 0;
+    sw::LapDiv lapdiv{};
+#endif
+};
+
+AdjPlan plan_adjoint(Prepared &pr, DeviceArena &arena, hipStream_t st)
+{
+    const Params &P = pr.P;
+    AdjPlan A;
+    const int R = pr.r;
+    const long long Ix = P.nx - 2 * R, Iz = P.nz - 2 * R;
+#if SW_DIM == 3
+    const long long Iy = P.ny - 2 * R;
+    const long long lines[3] = {Ix * Iy, Iz * Iy, Iz * Ix};
+#else
+    const long long lines[2] = {Ix, Iz};
+#endif
+    long long total = 0;
+    for (int f = 0; f < 2 * SW_DIM; f++)
+        total += P.bc[f] == 2 ? lines[f / 2] : 0;
+    if (total >= (1ll << 31))
+        fail("the adjoint's Neumann faces hold too many lines (%lld)", total);
+    A.halo_lines = (unsigned)total;
+#if SW_DIM == 3
+    set_lap_div(pr);
+    A.lapdiv = pr.lapdiv;
+    sw::Tiling &T = A.T;
+    T.ty = 64 / sw::kAdjRows * sw::kVec16;
+    T.txr = sw::kAdjRows;
+    T.gk = (int)((Iy + T.ty - 1) / T.ty);
+    T.gj = (int)((Ix + T.txr - 1) / T.txr);
+    T.ncols = T.gk * T.gj;
+    T.chunk = (T.ncols + 7) / 8;
+    T.nwords = P.nz / 32 + 3;
+    const long long pbytes = P.sz * (long long)sizeof(real_t);
+    // Planes per z chunk: short ones share halo rows in an XCD's L2 as the
+    // forward's do (220 x 316 x 316 so8: 4 planes 221 us, 2 226, 16 236), small
+    // grids take fewer to fill the chip (50 x 70 x 70 interior 12.8, 4 planes
+    // 14.3), deep queues and doubles a few more (160 x 220 x 240 so20 102, 4
+    // planes 108; float64 so8 148 and 153).
+    const int target = Iz * Ix * Iy < 1000 * 1000 ? 2 : !kF32 || R >= 8 ? 6 : 4;
+    const int zlen = (int)std::min<long long>(target, Iz);
+    T.zlen = zlen;
+    T.gz = (int)((Iz + zlen - 1) / zlen);
+    const long long blocks = 8ll * T.chunk * T.gz;
+    // 32-bit buffer offsets over the planes a tile touches
+    A.tiled = pbytes * (zlen + 2 * R + 1) < (1ll << 31) && P.ny >= sw::kVec16 &&
+              blocks + total / 64 + 1 < (1ll << 31) && !env_flag("SIMWAVE_HIP_UNTILED");
+    if (!A.tiled)
+        return A;
+    A.tiled_blocks = (int)blocks;
+    const long long words = (long long)T.ncols * T.nwords + 1;
+    unsigned *mask = arena.alloc<unsigned>((size_t)words);
+    hipLaunchKernelGGL(sw::k_zero_u32,
+                       dim3((unsigned)std::min<long long>((words + 255) / 256, 4096)), dim3(256),
+                       0, st, mask, words);
+    T.dmask = mask;
+    hipLaunchKernelGGL(sw::k_damp_flags, dim3(T.ncols, P.nz), dim3(256), 0, st, P.e, P.nz, P.nx,
+                       P.ny, R, T.gk, T.ty, T.txr, T.nwords, mask, mask + words - 1);
+    hip_check(hipGetLastError(), "k_damp_flags launch");
+#else
+    (void)arena;
+    (void)st;
+#endif
+    return A;
+}
+
+// Reverse interior update of one step; GM: gradient terms it adds.
+template <int R, int GM>
+void adj_update(const Params &P, const AdjPlan &L, hipStream_t st, LaunchTimer tm,
+                const sw::AdjArgs &A)
 {
 #if SW_DIM == 3
-    switch (P.r) {
-#define SW_ADJ_CASE(R)                                                              \
-    case R:                                                                         \
-        adj_update_z<R>(P, st, tm, vel, ub, W, ub1, ub2, u0, u1, u2, gacc, image);  \
+    if (L.tiled) {
+        launch_timed(sw::k_adj_update_tiled<R, GM>,
+                     dim3(L.tiled_blocks + (L.halo_lines + 63) / 64), dim3(64), st, tm, P,
+                     L.lapdiv, A, L.T, L.tiled_blocks);
         return;
-    SW_ADJ_CASE(1) SW_ADJ_CASE(2) SW_ADJ_CASE(3) SW_ADJ_CASE(4) SW_ADJ_CASE(5)
-    SW_ADJ_CASE(6) SW_ADJ_CASE(7) SW_ADJ_CASE(8) SW_ADJ_CASE(9) SW_ADJ_CASE(10)
-#undef SW_ADJ_CASE
-    default:
-        break;
     }
+    launch_timed(sw::k_adj_update<R, GM>, sw::adj_grid(P), sw::adj_block(), st, tm, P, A);
+    if (L.halo_lines)
+        hipLaunchKernelGGL((sw::k_adj_halo<R>), dim3((L.halo_lines + 255) / 256), dim3(256), 0,
+                           st, P, A);
 #else
-    switch (P.r) {
-#define SW_ADJ_CASE(R)                                                              \
-    case R:                                                                         \
-        launch_timed(sw::k_adj_update_z2d<R>,                                      \
-                     dim3((unsigned)((P.nx + 255) / 256),                           \
-                          (unsigned)((P.nz + sw::kAdjZChunk - 1) / sw::kAdjZChunk)), \
-                     dim3(256), st, tm, P, vel, ub, W, ub1, ub2, u0, u1, u2, gacc, image); \
-        return;
-    SW_ADJ_CASE(1) SW_ADJ_CASE(2) SW_ADJ_CASE(3) SW_ADJ_CASE(4) SW_ADJ_CASE(5)
-    SW_ADJ_CASE(6) SW_ADJ_CASE(7) SW_ADJ_CASE(8) SW_ADJ_CASE(9) SW_ADJ_CASE(10)
-#undef SW_ADJ_CASE
-    default:
-        break;
-    }
+    const int gx = (P.nx - 2 * R + 255) / 256, zlen = adj_zlen_2d(P, R);
+    const int blocks = gx * ((P.nz - 2 * R + zlen - 1) / zlen);
+    launch_timed(sw::k_adj_update_z2d<R, GM>, dim3(blocks + (L.halo_lines + 255) / 256),
+                 dim3(256), st, tm, P, A, zlen, gx, blocks);
 #endif
-    hipLaunchKernelGGL(sw::k_adj_update, sw::adj_grid(P), sw::adj_block(), 0, st, P, vel, ub, W,
-                       ub1, ub2, u0, u1, u2, gacc, image);
 }
+
+template <int GM>
+void adj_update(const Params &P, const AdjPlan &L, hipStream_t st, LaunchTimer tm,
+                const sw::AdjArgs &A)
+{
+    switch (P.r) {
+    case 1: return adj_update<1, GM>(P, L, st, tm, A);
+    case 2: return adj_update<2, GM>(P, L, st, tm, A);
+    case 3: return adj_update<3, GM>(P, L, st, tm, A);
+    case 4: return adj_update<4, GM>(P, L, st, tm, A);
+    case 5: return adj_update<5, GM>(P, L, st, tm, A);
+    case 6: return adj_update<6, GM>(P, L, st, tm, A);
+    case 7: return adj_update<7, GM>(P, L, st, tm, A);
+    case 8: return adj_update<8, GM>(P, L, st, tm, A);
+    case 9: return adj_update<9, GM>(P, L, st, tm, A);
+    default: return adj_update<10, GM>(P, L, st, tm, A);
+    }
+}
+#endif
 
 // Shot record and its adjoint: runs the forward of a constant-density shot
 // (device arrays, as the device entry; stride 0, steps 1..T) saving the two
@@ -2693,20 +2771,21 @@ double run_adjoint(const Args &a, const real_t *rec_adj, double *grad, real_t *g
     if (store_all)
         K = T;
     const size_t ncp = store_all ? 1 : (T + K - 1) / K;
+    const size_t m_last = (ncp - 1) * K;      // first level of the last segment
     const int nb = (int)std::min<long long>(((long long)npts + 255) / 256, 16384);
     auto zero = [&](real_t *p, size_t count) {
         hipLaunchKernelGGL(sw::k_fill, dim3(nb), dim3(256), 0, st, p, (long long)count,
                            (real_t)0);
     };
+    const AdjPlan launch = plan_adjoint(pr, arena, st);
     real_t *cp = store_all ? nullptr : arena.alloc<real_t>(2 * ncp * npts);
     real_t *seg = arena.alloc<real_t>((K + 2) * npts);
-    real_t *ubar = arena.alloc<real_t>(3 * npts);
-    real_t *W = arena.alloc<real_t>(npts);
+    real_t *lam = arena.alloc<real_t>(2 * npts);    // l^k in lam + (k % 2) npts
+    real_t *W = arena.alloc<real_t>(2 * npts);      // c l^k, likewise
     // the reverse steps add their gradient terms here, in the working
     // precision; every kGradFlush steps (counted over the whole sweep, so
     // the sums do not depend on K) and at the end they go into grad
     real_t *gacc = arena.alloc<real_t>(npts);
-    size_t reverse_steps = 0;
     // the forward's coefficient C = q / den per point
     real_t *Cq = arena.alloc<real_t>(npts);
     hipLaunchKernelGGL(sw::k_scaled_q, dim3(nb), dim3(256), 0, st, P.q, P.e, Cq,
@@ -2716,10 +2795,15 @@ double run_adjoint(const Args &a, const real_t *rec_adj, double *grad, real_t *g
                            (long long)npts);
     };
     // the shot starts from rest whatever the caller's slots hold, so that
-    // the all-levels and checkpointed sweeps see the same initial state
+    // the all-levels and checkpointed sweeps see the same initial state; the
+    // steps write the interior and Neumann mirrors only, so every level's
+    // buffer starts as zeros
     zero(a.u, 3 * npts);
     zero(seg, (K + 2) * npts);
-    zero(ubar, 3 * npts);
+    if (cp)
+        zero(cp, 2 * ncp * npts);
+    zero(lam, 2 * npts);
+    zero(W, 2 * npts);
     zero(gacc, npts);
     hipLaunchKernelGGL(sw::k_fill_f64, dim3(nb), dim3(256), 0, st, grad, (long long)npts);
     if (gw && a.nsrc)
@@ -2727,41 +2811,37 @@ double run_adjoint(const Args &a, const real_t *rec_adj, double *grad, real_t *g
                            (long long)(T * a.nsrc), (real_t)0);
     hip_check(hipGetLastError(), "adjoint set-up");
 
-    // forward with checkpoints
-    std::vector<StepSlots> plan = plan_slots(a);
+    // The forward writes each level where the reverse sweep wants it: the two
+    // levels that open a checkpoint segment into the checkpoints, the rest of
+    // the last segment into `seg` (it needs no recomputation), the others into
+    // the caller's rotating slots.  Plan entries name levels.
     real_t *u = a.u;
-    auto slot_ptr = [&](size_t sl) { return u + sl * npts; };
-    auto save = [&](size_t idx) {
-        if (idx % K)
-            return;
-        const StepSlots &s = plan[idx];
-        const size_t j = idx / K;
-        hip_check(hipMemcpyAsync(cp + (2 * j) * npts, slot_ptr(s.prev), npts * sizeof(real_t),
-                                 hipMemcpyDeviceToDevice, st), "checkpoint");
-        hip_check(hipMemcpyAsync(cp + (2 * j + 1) * npts, slot_ptr(s.cur),
-                                 npts * sizeof(real_t), hipMemcpyDeviceToDevice, st),
-                  "checkpoint");
+    auto checkpoint_ptr = [&](size_t l) {     // l % K is 0 or 1
+        return cp + (K == 1 ? l : 2 * (l / K) + l % K) * npts;
+    };
+    auto forward_ptr = [&](size_t l) {
+        if (!store_all && l <= m_last + 1 && (K == 1 || l % K < 2))
+            return checkpoint_ptr(l);
+        return l >= m_last ? seg + (l - m_last) * npts : u + l % 3 * npts;
+    };
+    size_t m = m_last;                        // first level of the segment in `seg`
+    auto level_ptr = [&](size_t l) {
+        const bool saved = !store_all && (l <= m + 1 || (m != m_last && l >= m + K));
+        return saved ? checkpoint_ptr(l) : seg + (l - m) * npts;
     };
     auto nop = [](size_t) {};
     auto noswap = [](size_t, size_t) {};
     auto no_uploads = [](size_t) { return false; };
-    auto seg_ptr = [&](size_t l) { return seg + l * npts; };
-    if (store_all) {
-        // level l of the run in seg + l*npts
-        std::vector<StepSlots> sp;
-        for (size_t n = 1; n <= T; n++)
-            sp.push_back(StepSlots{n - 1, n, n + 1, false, 0, 0});
-        time_loop(a, pr, sp, 0, sp.size(), a.receivers, 0, flags & kFlagOverlapReceivers, st,
-                  seg_ptr, nop, nop, noswap, no_uploads);
-        // the caller's slots end as after a plain forward: level l in l % 3
-        for (size_t l = T - 1; l <= T + 1; l++)
-            hip_check(hipMemcpyAsync(slot_ptr(l % 3), seg_ptr(l), npts * sizeof(real_t),
-                                     hipMemcpyDeviceToDevice, st),
-                      "final levels");
-    } else {
-        time_loop(a, pr, plan, 0, plan.size(), a.receivers, 0, flags & kFlagOverlapReceivers,
-                  st, slot_ptr, save, nop, noswap, no_uploads);
-    }
+    std::vector<StepSlots> plan;
+    for (size_t n = 1; n <= T; n++)
+        plan.push_back(StepSlots{n - 1, n, n + 1, false, 0, 0});
+    time_loop(a, pr, plan, 0, T, a.receivers, 0, flags & kFlagOverlapReceivers, st, forward_ptr,
+              nop, nop, noswap, no_uploads);
+    // the caller's slots end as after a plain forward: level l in l % 3
+    for (size_t l = T - 1; l <= T + 1; l++)
+        hip_check(hipMemcpyAsync(u + l % 3 * npts, level_ptr(l), npts * sizeof(real_t),
+                                 hipMemcpyDeviceToDevice, st),
+                  "final levels");
     if ((flags & kAdjResidual) && a.nrec) {
         // the shot record rows 0 .. T-1 are complete on `st`
         real_t *res = arena.alloc<real_t>(T * a.nrec);
@@ -2794,68 +2874,68 @@ double run_adjoint(const Args &a, const real_t *rec_adj, double *grad, real_t *g
     // backward over the checkpoint segments
     Args seg_args = a;
     seg_args.nrec = 0;
+    size_t reverse_steps = 0;
+    bool pending = false;       // the last step's gradient term is to be added
     for (size_t j = ncp; j-- > 0;) {
-        const size_t m = j * K;                   // levels m, m+1 saved
+        m = j * K;                                // levels m, m+1 saved
         const size_t n_lo = m + 1, n_hi = std::min(m + K, T);
-        if (!store_all) {
-            hip_check(hipMemcpyAsync(seg, cp + (2 * j) * npts, 2 * npts * sizeof(real_t),
-                                     hipMemcpyDeviceToDevice, st),
-                      "restore checkpoint");
-            std::vector<StepSlots> sp;
-            for (size_t n = n_lo; n <= n_hi; n++)
-                sp.push_back(StepSlots{n - 1 - m, n - m, n + 1 - m, false, 0, 0});
-            seg_args.n0 = n_lo;
-            seg_args.n1 = n_hi;
-            time_loop(seg_args, pr, sp, 0, sp.size(), nullptr, 0, 0u, st, seg_ptr, nop, nop,
-                      noswap, no_uploads);
-        }
+        if (m != m_last && K > 2)     // levels m+2 .. m+K-1; the next segment opens with m+K
+            time_loop(seg_args, pr, plan, m, m + K - 2, nullptr, 0, 0u, st, level_ptr, nop,
+                      nop, noswap, no_uploads);
         for (size_t n = n_hi; n >= n_lo; n--) {
             const size_t k = n + 1;
-            real_t *ub = ubar + (k % 3) * npts;
-            real_t *ub1 = ubar + ((k - 1) % 3) * npts;
-            real_t *ub2 = ubar + ((k - 2) % 3) * npts;
-            if (k <= T && a.nrec && rg.nu)
+            real_t *l = lam + (k % 2) * npts, *Wk = W + (k % 2) * npts;
+            if (k <= T && a.nrec && rg.nu) {
                 hipLaunchKernelGGL(sw::k_adj_rec_gather, dim3((unsigned)((rg.nu + 255) / 256)),
-                                   dim3(256), 0, st, rg.pts, rg.start, rg.cnt, rg.nu, rg.qs,
-                                   rg.ws, rec_adj + (k - 1) * a.nrec, ub);
-            else if (k <= T && a.nrec)
+                                   dim3(256), 0, st, P, Cq, rg.pts, rg.start, rg.cnt, rg.nu,
+                                   rg.qs, rg.ws, rec_adj + (k - 1) * a.nrec, l, Wk);
+            } else if (k <= T && a.nrec) {
                 hipLaunchKernelGGL(sw::k_adj_receivers, dim3((unsigned)a.nrec), dim3(256), 0,
                                    st, P, pr.rbox, pr.rw, (int)a.nrec,
-                                   rec_adj + (k - 1) * a.nrec, ub);
+                                   rec_adj + (k - 1) * a.nrec, l);
+                hipLaunchKernelGGL(sw::k_adj_cw, sw::adj_grid(P), sw::adj_block(), 0, st, P, Cq,
+                                   l, Wk);
+            }
 #if SW_DIM == 3
             const int axes[3] = {0, 1, 2};
             const long long lines[3] = {
                 (long long)(P.nx - 2 * r) * (P.ny - 2 * r),
                 (long long)(P.nz - 2 * r) * (P.ny - 2 * r),
                 (long long)(P.nz - 2 * r) * (P.nx - 2 * r)};
-            const int nph = 3;
 #else
             const int axes[2] = {0, 2};
             const long long lines[2] = {(long long)(P.nx - 2 * r), (long long)(P.nz - 2 * r)};
-            const int nph = 2;
 #endif
-            for (int ph = 0; ph < nph; ph++)   // z first: the reverse of y, x, z
-                hipLaunchKernelGGL(sw::k_adj_bc_phase,
-                                   dim3((unsigned)((lines[ph] + 255) / 256)), dim3(256), 0, st,
-                                   P, ub, axes[ph]);
-            hipLaunchKernelGGL(sw::k_adj_cw, sw::adj_grid(P), sw::adj_block(), 0, st, P, Cq, ub,
-                               W);
+            for (int ph = 0; ph < SW_DIM; ph++)   // z first: the reverse of y, x, z
+                if (P.bc[2 * ph] == 2 || P.bc[2 * ph + 1] == 2)
+                    hipLaunchKernelGGL(sw::k_adj_bc_phase,
+                                       dim3((unsigned)((lines[ph] + 255) / 256)), dim3(256), 0,
+                                       st, P, Cq, l, Wk, axes[ph]);
             if (a.nsrc && gw)
                 hipLaunchKernelGGL(sw::k_adj_sources, dim3((unsigned)a.nsrc), dim3(256), 0, st,
-                                   P, ub, gw + (n - 1) * a.nsrc);
-            const bool timed = utime.used + 2 <= utime.ev.size();
+                                   P, l, gw + (n - 1) * a.nsrc);
             LaunchTimer tm;
-            if (timed) {
+            if (utime.used + 2 <= utime.ev.size()) {
                 tm = LaunchTimer{utime.ev[utime.used], utime.ev[utime.used + 1]};
                 utime.used += 2;
             }
-            adj_update(P, st, tm, a.vel, ub, W, ub1, ub2, seg + (n + 1 - m) * npts,
-                       seg + (n - m) * npts, seg + (n - 1 - m) * npts, gacc, image ? 1 : 0);
-            if (++reverse_steps % kGradFlush == 0)
+            sw::AdjArgs A{a.vel, Cq, l, Wk, lam + ((k + 1) % 2) * npts,
+                          W + ((k + 1) % 2) * npts, {}, gacc, image ? 1 : 0};
+            for (size_t t = pending ? 0 : 1; t < 4; t++)
+                A.u[t] = level_ptr(n + 2 - t);
+            const bool flush = ++reverse_steps % kGradFlush == 0;
+            if (pending) {
+                adj_update<2>(P, launch, st, tm, A);
+                pending = false;
+            } else if (flush || n == n_lo) {
+                adj_update<1>(P, launch, st, tm, A);
+            } else {
+                adj_update<0>(P, launch, st, tm, A);
+                pending = true;
+            }
+            if (flush)
                 flush_grad();
             hip_check(hipGetLastError(), "adjoint step");
-            if (n == n_lo)
-                break;
         }
     }
     flush_grad();
