@@ -1459,8 +1459,9 @@ int simwave_hip_last_timings(double *out, int n);
 const char *simwave_hip_variant(void);
 /* No reference counterpart.  Hands the freed memory that the current
  * device's default pool keeps for reuse (the library's stream-ordered
- * allocations; up to 8 GiB is kept between runs) back to the device, after
- * waiting for the device, so that a free-memory query sees it.  0, or -1. */
+ * allocations; up to 8 GiB is kept between runs) and the gradient entries'
+ * kept blocks (up to 8 GiB more) back to the device, after waiting for the
+ * device, so that a free-memory query sees it.  0, or -1. */
 int simwave_hip_trim_pool(void);
 
 /* No reference counterpart (the reference's forward takes host arrays

@@ -160,6 +160,11 @@ constexpr long long kOverlapMinPoints = 1ll << 22;
 // quietly keeps its receivers on its one stream.
 extern "C" int simwave_hip_overlap_acquire(void);
 extern "C" void simwave_hip_overlap_release(void);
+extern "C" void *simwave_hip_block_take(int device, unsigned long long bytes,
+                                        unsigned long long *got);
+extern "C" int simwave_hip_block_put(int device, void *p, unsigned long long bytes,
+                                     unsigned long long limit);
+extern "C" void *simwave_hip_block_evict(int device, unsigned long long limit);
 
 struct OverlapLease {
     bool held = false;
@@ -299,10 +304,59 @@ struct DeviceArena {
     std::vector<void *> ptrs;
     char *base = nullptr;
     size_t cap = 0, used = 0;
+    // Blocks kept from one run for the next (keep_blocks): the run's own list,
+    // those it released on the way free for its later requests (one stream, so
+    // in order).
+    struct Block {
+        void *p;
+        size_t bytes;
+        bool free;
+    };
+    int keep_device = -1;
+    std::vector<Block> blocks;
     explicit DeviceArena(hipStream_t s) : stream(s) {}
     DeviceArena(hipStream_t s, void *region, size_t bytes)
         : stream(s), base(static_cast<char *>(region)), cap(bytes)
     {
+    }
+    // From here on requests of kKeepMin bytes and more are served from blocks
+    // that outlive the run: hipMallocAsync and hipFreeAsync map and unmap
+    // them, 30 us and up to 3 ms each on the host (a gradient of 200 x 220 x
+    // 240 points spent 4.4 of its 16.4 ms so).  At most kPoolKeepBytes per
+    // device are kept, the oldest go first, and simwave_hip_trim_pool gives all
+    // of them back.
+    static constexpr size_t kKeepMin = 1u << 20;
+    void keep_blocks() { hip_check(hipGetDevice(&keep_device), "hipGetDevice"); }
+    void *alloc_block(size_t bytes)
+    {
+        for (Block &b : blocks)
+            if (b.free && b.bytes >= bytes && b.bytes - bytes <= bytes / 4) {
+                b.free = false;
+                return b.p;
+            }
+        blocks.reserve(blocks.size() + 1);
+        unsigned long long got = bytes;
+        void *p = simwave_hip_block_take(keep_device, bytes, &got);
+        if (!p) {
+            hipError_t e = hipMallocAsync(&p, bytes, stream);
+            if (e == hipErrorOutOfMemory && drop_blocks(keep_device, 0, stream)) {
+                hip_check(hipStreamSynchronize(stream), "kept blocks");
+                e = hipMallocAsync(&p, bytes, stream);
+            }
+            hip_check(e, "hipMallocAsync");
+        }
+        blocks.push_back({p, (size_t)got, false});
+        return p;
+    }
+    // Frees the oldest kept blocks until at most `limit` bytes are left.
+    static bool drop_blocks(int device, unsigned long long limit, hipStream_t st)
+    {
+        bool any = false;
+        while (void *p = simwave_hip_block_evict(device, limit)) {
+            (void)hipFreeAsync(p, st);
+            any = true;
+        }
+        return any;
     }
     template <typename T>
     T *alloc(size_t count)
@@ -319,6 +373,8 @@ struct DeviceArena {
             used += bytes;
             return static_cast<T *>(p);
         }
+        if (keep_device >= 0 && count * sizeof(T) >= kKeepMin)
+            return static_cast<T *>(alloc_block(count * sizeof(T)));
         void *p = nullptr;
         hip_check(hipMallocAsync(&p, count * sizeof(T), stream), "hipMallocAsync");
         ptrs.push_back(p);
@@ -326,18 +382,18 @@ struct DeviceArena {
     }
     void release(void *p)
     {
+        for (Block &b : blocks)
+            if (b.p == p) {
+                b.free = true;
+                return;
+            }
         auto it = std::find(ptrs.begin(), ptrs.end(), p);
         if (it != ptrs.end()) {
             (void)hipFreeAsync(p, stream);
             ptrs.erase(it);
         }
     }
-    ~DeviceArena()
-    {
-        for (void *p : ptrs)
-            (void)hipFreeAsync(p, stream);
-        (void)hipStreamSynchronize(stream);
-    }
+    ~DeviceArena();
 };
 
 // Freed stream-ordered allocations stay in the device's default pool up to
@@ -345,6 +401,22 @@ struct DeviceArena {
 // new mappings; beyond it the pool returns memory to the device at the next
 // synchronisation, where other allocators (PyTorch's) can use it.
 constexpr uint64_t kPoolKeepBytes = 8ull << 30;
+
+DeviceArena::~DeviceArena()
+{
+    for (void *p : ptrs)
+        (void)hipFreeAsync(p, stream);
+    // kept blocks may serve any stream next: only once this one is done
+    const bool done = hipStreamSynchronize(stream) == hipSuccess;
+    for (const Block &b : blocks) {
+        if (done && b.bytes <= kPoolKeepBytes) {
+            drop_blocks(keep_device, kPoolKeepBytes - b.bytes, stream);
+            if (simwave_hip_block_put(keep_device, b.p, b.bytes, kPoolKeepBytes))
+                continue;
+        }
+        (void)hipFreeAsync(b.p, stream);
+    }
+}
 
 bool default_pool(hipMemPool_t &pool)
 {
@@ -2759,6 +2831,7 @@ double run_adjoint(const Args &a, const real_t *rec_adj, double *grad, real_t *g
         }
     } trim;
     DeviceArena arena(st);
+    arena.keep_blocks();
     Prepared pr = prepare(a, true, 0u, arena, st);
     if (pr.halo_sources)
         fail("the adjoint needs every source box inside the interior");
@@ -3375,6 +3448,9 @@ SW_EXPORT int simwave_hip_trim_pool(void)
         hipMemPool_t pool;
         if (!default_pool(pool))
             fail("no default memory pool on the current device");
+        int dev = 0;
+        hip_check(hipGetDevice(&dev), "hipGetDevice");
+        DeviceArena::drop_blocks(dev, 0, nullptr);
         hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");
         hip_check(hipMemPoolTrimTo(pool, 0), "hipMemPoolTrimTo");
         return 0.0;
