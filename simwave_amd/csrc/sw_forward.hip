@@ -902,9 +902,10 @@ bool prefer_zmarch(const Prepared &pr)
 // for sources and boundaries; so16 160 against 232 us).  Otherwise from 2 M
 // interior points on: float32 from radius 3 (276^3 so8: 185 us, z-marching
 // 275; so16 220 against 317; 148^3 so8 38 against 54; 116^3 29 against 30;
-// but 220^3 so2 100 against 80, so4 104 against 105), float64 from radius 2
-// (220^3 so4 170 against 227, so8 171 against 344, so16 234 against k_step3d's
-// 459).  A caller-owned arena (the allocation-free entry) has no room
+// but 220^3 so2 100 against 80), radius 2 from 12 M points (240^3 so4 128
+// against 133, 276^3 184 against 196; 220^3 104 against 105), float64 from
+// radius 2 (220^3 so4 170 against 227, so8 171 against 344, so16 234 against
+// k_step3d's 459).  A caller-owned arena (the allocation-free entry) has no room
 // for the packed coefficients.
 bool prefer_tiled_vd(const Prepared &pr, bool oblong, const DeviceArena &arena)
 {
@@ -913,7 +914,8 @@ bool prefer_tiled_vd(const Prepared &pr, bool oblong, const DeviceArena &arena)
     const char *tile = getenv("SIMWAVE_HIP_TILE");
     if ((tile && *tile) || oblong)
         return true;
-    return pr.r >= (kF32 ? 3 : 2) && interior_points(pr) >= 2ll * 1000 * 1000;
+    const long long least = kF32 && pr.r == 2 ? 12 : 2;   // million points
+    return pr.r >= 2 && interior_points(pr) >= least * 1000 * 1000;
 }
 
 template <int R, int WR, int RPT, int NW, int V, bool D64, int RHO>
@@ -1004,9 +1006,14 @@ TiledKernel tiled_entry(int v)
     // 8 rows of 8-byte lanes with 2 rows per lane up to radius 5 (float64: 4),
     // above it 8 rows of 16-byte lanes, whose one row per lane keeps the z
     // queue short (276^3 so8: 185 against 196 us; so16 224 against 220, 220^3
-    // so20 200 against 191; float64 so16 257 against 234)
+    // so20 200 against 191; float64 so16 257 against 234); radius 2 half the
+    // rows, twice as wide (160 x 200 x 271 so4: 92 against 94 us, 240^3 128
+    // against 133; float64 155 against 164 and 199 against 211; radius 4 148
+    // against 142 at 190 x 240 x 270)
     (void)v;
-    if constexpr (R <= (kF32 ? 5 : 4))
+    if constexpr (R == 2)
+        return tiled_config<R, 2, 2, 1, sw::kVec8>();
+    else if constexpr (R <= (kF32 ? 5 : 4))
         return tiled_config<R, 4, 2, 1, sw::kVec8>();
     else
         return tiled_config<R, 8, 1, 1, sw::kVec16>();

@@ -71,3 +71,17 @@ def test_subnormal_quotients(gpu, density, scale, monkeypatch):
     kw["wavelet"] = np.zeros_like(kw["wavelet"])
     (u_h, r_h), (u_o, r_o) = _forward(kw, "hip"), _forward(kw, "oracle")
     assert np.any(u_o) and np.array_equal(u_h, u_o) and np.array_equal(r_h, r_o)
+
+
+@pytest.mark.parametrize("dtype", [F32, F64], ids=["f32", "f64"])
+@pytest.mark.parametrize("shape", [(19, 8, 133), (13, 67, 67), (12, 131, 20)])
+def test_radius2_tiles(gpu, shape, dtype, monkeypatch):
+    """Radius 2 has a tile of its own: 4 rows, 64 points (float64 32)."""
+    print("radius 2 tiles", shape, np.dtype(dtype).name, flush=True)
+    monkeypatch.setenv("SIMWAVE_HIP_TILE", "0")
+    setup = cases.make_case(dim=3, density=True, tf=0.05, shape=shape, space_order=4, dtype=dtype,
+                            bc=BC, window=3)
+    u_h, r_h = harness.run(setup, "hip")
+    assert _step_kernel_of_last_run(3, "vd", "f64" if dtype is F64 else "f32") == 1
+    u_o, r_o = harness.run(setup, "oracle")
+    assert np.array_equal(u_h, u_o) and np.array_equal(r_h, r_o)
