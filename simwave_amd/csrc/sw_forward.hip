@@ -295,6 +295,8 @@ std::vector<Box> make_boxes(const char *what, size_t count, const size_t *iv,
     return boxes;
 }
 
+bool default_pool(hipMemPool_t &pool);
+
 // Stream-ordered device allocations released when the object dies.  With a
 // base pointer it instead hands out consecutive 256-byte aligned pieces of
 // that caller-owned region (no allocation, nothing to free) and fails once
@@ -340,7 +342,11 @@ struct DeviceArena {
         if (!p) {
             hipError_t e = hipMallocAsync(&p, bytes, stream);
             if (e == hipErrorOutOfMemory && drop_blocks(keep_device, 0, stream)) {
+                (void)hipGetLastError();
                 hip_check(hipStreamSynchronize(stream), "kept blocks");
+                hipMemPool_t pool;
+                if (default_pool(pool))
+                    (void)hipMemPoolTrimTo(pool, 0);
                 e = hipMallocAsync(&p, bytes, stream);
             }
             hip_check(e, "hipMallocAsync");
