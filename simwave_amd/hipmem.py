@@ -30,18 +30,26 @@ _SIGS = {
     "simwave_hip_event_synchronize": [_VP],
     "simwave_hip_event_destroy": [_VP],
 }
-_BOUND = set()
-_BIND_LOCK = threading.Lock()
+# re-entrant: a collection inside may free an array of this module
+_BIND_LOCK = threading.RLock()
 
 
 def _fn(lib, name):
-    key = (id(lib), name)
-    fn = getattr(lib, name)
-    if key not in _BOUND:
+    """The library's entry point `name` with its argument types set: a function
+    object of this module's own (lib[name], kept on the library handle), typed
+    before any other thread sees it and never typed again, since argument types
+    set anew are freed under another thread's call."""
+    fns = lib.__dict__.get("_hipmem_fns")
+    fn = fns.get(name) if fns else None
+    if fn is None:
         with _BIND_LOCK:
-            fn.argtypes = _SIGS[name]
-            fn.restype = ctypes.c_int
-            _BOUND.add(key)
+            fns = lib.__dict__.setdefault("_hipmem_fns", {})
+            fn = fns.get(name)
+            if fn is None:
+                fn = lib[name]
+                fn.argtypes = _SIGS[name]
+                fn.restype = ctypes.c_int
+                fns[name] = fn
     return fn
 
 
