@@ -62,6 +62,13 @@ SW_COMMON_EXPORT int simwave_hip_overlap_holders(void)
     return g_overlap_holders.load();
 }
 
+// Bytes that `device` holds in kept blocks.
+SW_COMMON_EXPORT unsigned long long simwave_hip_block_held(int device)
+{
+    std::lock_guard<std::mutex> g(g_blocks_mutex);
+    return kept_bytes(device);
+}
+
 // The smallest kept block of `device` that holds `bytes` and is at most a
 // quarter larger, taken off the list (its size in *got), or null.
 SW_COMMON_EXPORT void *simwave_hip_block_take(int device, unsigned long long bytes,

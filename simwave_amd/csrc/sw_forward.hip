@@ -15,6 +15,7 @@
 // slots of HBM, and the even-stride content exchange becomes a swap of the two
 // device pointers.
 #include "sw_kernels.hpp"
+#include "sw_memory.hpp"
 #include "sw_step3d.hpp"
 #include "sw_adjoint.hpp"
 #include "sw_batch.hpp"
@@ -160,6 +161,7 @@ constexpr long long kOverlapMinPoints = 1ll << 22;
 // quietly keeps its receivers on its one stream.
 extern "C" int simwave_hip_overlap_acquire(void);
 extern "C" void simwave_hip_overlap_release(void);
+extern "C" unsigned long long simwave_hip_block_held(int device);
 extern "C" void *simwave_hip_block_take(int device, unsigned long long bytes,
                                         unsigned long long *got);
 extern "C" int simwave_hip_block_put(int device, void *p, unsigned long long bytes,
@@ -295,141 +297,72 @@ std::vector<Box> make_boxes(const char *what, size_t count, const size_t *iv,
     return boxes;
 }
 
-bool default_pool(hipMemPool_t &pool);
-
-// Stream-ordered device allocations released when the object dies.  With a
-// base pointer it instead hands out consecutive 256-byte aligned pieces of
-// that caller-owned region (no allocation, nothing to free) and fails once
-// `cap` bytes are used.
-struct DeviceArena {
-    hipStream_t stream;
-    std::vector<void *> ptrs;
-    char *base = nullptr;
-    size_t cap = 0, used = 0;
-    // Blocks kept from one run for the next (keep_blocks): the run's own list,
-    // those it released on the way free for its later requests (one stream, so
-    // in order).
-    struct Block {
-        void *p;
-        size_t bytes;
-        bool free;
-    };
-    int keep_device = -1;
-    std::vector<Block> blocks;
-    explicit DeviceArena(hipStream_t s) : stream(s) {}
-    DeviceArena(hipStream_t s, void *region, size_t bytes)
-        : stream(s), base(static_cast<char *>(region)), cap(bytes)
-    {
-    }
-    // From here on requests of kKeepMin bytes and more are served from blocks
-    // that outlive the run: hipMallocAsync and hipFreeAsync map and unmap
-    // them, 30 us and up to 3 ms each on the host (a gradient of 200 x 220 x
-    // 240 points spent 4.4 of its 16.4 ms so).  At most kPoolKeepBytes per
-    // device are kept, the oldest go first, and simwave_hip_trim_pool gives all
-    // of them back.
-    static constexpr size_t kKeepMin = 1u << 20;
-    void keep_blocks() { hip_check(hipGetDevice(&keep_device), "hipGetDevice"); }
-    void *alloc_block(size_t bytes)
-    {
-        for (Block &b : blocks)
-            if (b.free && b.bytes >= bytes && b.bytes - bytes <= bytes / 4) {
-                b.free = false;
-                return b.p;
-            }
-        blocks.reserve(blocks.size() + 1);
-        unsigned long long got = bytes;
-        void *p = simwave_hip_block_take(keep_device, bytes, &got);
-        if (!p) {
-            hipError_t e = hipMallocAsync(&p, bytes, stream);
-            if (e == hipErrorOutOfMemory && drop_blocks(keep_device, 0, stream)) {
-                (void)hipGetLastError();
-                hip_check(hipStreamSynchronize(stream), "kept blocks");
-                hipMemPool_t pool;
-                if (default_pool(pool))
-                    (void)hipMemPoolTrimTo(pool, 0);
-                e = hipMallocAsync(&p, bytes, stream);
-            }
-            hip_check(e, "hipMallocAsync");
-        }
-        blocks.push_back({p, (size_t)got, false});
-        return p;
-    }
-    // Frees the oldest kept blocks until at most `limit` bytes are left.
-    static bool drop_blocks(int device, unsigned long long limit, hipStream_t st)
-    {
-        bool any = false;
-        while (void *p = simwave_hip_block_evict(device, limit)) {
-            (void)hipFreeAsync(p, st);
-            any = true;
-        }
-        return any;
-    }
-    template <typename T>
-    T *alloc(size_t count)
-    {
-        if (count == 0)
-            return nullptr;
-        if (base) {
-            const size_t bytes = (count * sizeof(T) + 255) / 256 * 256;
-            if (bytes > cap - used)
-                fail("the run needs more than the %zu bytes of the library's static "
-                     "scratch (%zu used before a request of %zu bytes); use the "
-                     "allocating entry point for this grid", cap, used, count * sizeof(T));
-            void *p = base + used;
-            used += bytes;
-            return static_cast<T *>(p);
-        }
-        if (keep_device >= 0 && count * sizeof(T) >= kKeepMin)
-            return static_cast<T *>(alloc_block(count * sizeof(T)));
-        void *p = nullptr;
-        hip_check(hipMallocAsync(&p, count * sizeof(T), stream), "hipMallocAsync");
-        ptrs.push_back(p);
-        return static_cast<T *>(p);
-    }
-    void release(void *p)
-    {
-        for (Block &b : blocks)
-            if (b.p == p) {
-                b.free = true;
-                return;
-            }
-        auto it = std::find(ptrs.begin(), ptrs.end(), p);
-        if (it != ptrs.end()) {
-            (void)hipFreeAsync(p, stream);
-            ptrs.erase(it);
-        }
-    }
-    ~DeviceArena();
-};
-
-// Freed stream-ordered allocations stay in the device's default pool up to
-// this many bytes, so repeated runs of one grid reuse their memory without
-// new mappings; beyond it the pool returns memory to the device at the next
-// synchronisation, where other allocators (PyTorch's) can use it.
-constexpr uint64_t kPoolKeepBytes = 8ull << 30;
-
-DeviceArena::~DeviceArena()
-{
-    for (void *p : ptrs)
-        (void)hipFreeAsync(p, stream);
-    // kept blocks may serve any stream next: only once this one is done
-    const bool done = hipStreamSynchronize(stream) == hipSuccess;
-    for (const Block &b : blocks) {
-        if (done && b.bytes <= kPoolKeepBytes) {
-            drop_blocks(keep_device, kPoolKeepBytes - b.bytes, stream);
-            if (simwave_hip_block_put(keep_device, b.p, b.bytes, kPoolKeepBytes))
-                continue;
-        }
-        (void)hipFreeAsync(b.p, stream);
-    }
-}
-
 bool default_pool(hipMemPool_t &pool)
 {
     int dev = 0;
     return hipGetDevice(&dev) == hipSuccess &&
            hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess;
 }
+
+// The device calls of the arena (sw_memory.hpp).
+struct DeviceMemory {
+    typedef hipStream_t stream;
+    static int device()
+    {
+        int dev = -1;
+        hip_check(hipGetDevice(&dev), "hipGetDevice");
+        return dev;
+    }
+    // true, or false where the device is out of memory
+    static bool alloc(void **p, size_t bytes, hipStream_t st)
+    {
+        const hipError_t e = hipMallocAsync(p, bytes, st);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            return false;
+        }
+        hip_check(e, "hipMallocAsync");
+        return true;
+    }
+    static void free(void *p, hipStream_t st) { (void)hipFreeAsync(p, st); }
+    static bool synchronize(hipStream_t st) { return hipStreamSynchronize(st) == hipSuccess; }
+    static void trim()
+    {
+        hipMemPool_t pool;
+        if (default_pool(pool))
+            (void)hipMemPoolTrimTo(pool, 0);
+    }
+    static void *take(int device, size_t bytes, size_t *got)
+    {
+        unsigned long long n = bytes;
+        void *p = simwave_hip_block_take(device, bytes, &n);
+        *got = (size_t)n;
+        return p;
+    }
+    static bool put(int device, void *p, size_t bytes, size_t limit)
+    {
+        return simwave_hip_block_put(device, p, bytes, limit) != 0;
+    }
+    static void *evict(int device, size_t limit) { return simwave_hip_block_evict(device, limit); }
+    [[noreturn]] static void out_of_memory(size_t bytes)
+    {
+        fail("hipMallocAsync: out of memory (%zu bytes)", bytes);
+    }
+    [[noreturn]] static void region_full(size_t bytes, size_t cap, size_t used)
+    {
+        fail("the run needs more than the %zu bytes of the library's static "
+             "scratch (%zu used before a request of %zu bytes); use the "
+             "allocating entry point for this grid", cap, used, bytes);
+    }
+};
+
+using DeviceArena = sw::Arena<DeviceMemory>;
+
+// Freed stream-ordered allocations stay in the device's default pool up to
+// this many bytes, so repeated runs of one grid reuse their memory without
+// new mappings; beyond it the pool returns memory to the device at the next
+// synchronisation, where other allocators (PyTorch's) can use it.
+constexpr uint64_t kPoolKeepBytes = sw::kKeptBlockBytes;
 
 void keep_pool_memory()
 {
@@ -2835,12 +2768,16 @@ double run_adjoint(const Args &a, const real_t *rec_adj, double *grad, real_t *g
     keep_pool_memory();
     struct PoolTrim {
         // the sweep's levels and checkpoints are the largest allocations of
-        // the library: hand them back to the device once it has finished
+        // the library: what is above kPoolKeepBytes in kept blocks and pool
+        // together goes back to the device once it has finished
         ~PoolTrim()
         {
             hipMemPool_t pool;
-            if (default_pool(pool))
-                (void)hipMemPoolTrimTo(pool, kPoolKeepBytes);
+            int dev = 0;
+            if (!default_pool(pool) || hipGetDevice(&dev) != hipSuccess)
+                return;
+            const uint64_t held = std::min<uint64_t>(simwave_hip_block_held(dev), kPoolKeepBytes);
+            (void)hipMemPoolTrimTo(pool, kPoolKeepBytes - held);
         }
     } trim;
     DeviceArena arena(st);
@@ -3299,8 +3236,7 @@ SW_EXPORT int simwave_hip_device_alloc(unsigned long long bytes, void *stream, v
             fail("device_alloc: NULL result pointer");
         *ptr = nullptr;
         keep_pool_memory();
-        hip_check(hipMallocAsync(ptr, bytes ? bytes : 1, (hipStream_t)stream),
-                  "hipMallocAsync");
+        *ptr = DeviceArena::fresh(bytes ? bytes : 1, (hipStream_t)stream);
         return 0.0;
     });
     return r < 0 ? -1 : 0;
@@ -3463,7 +3399,7 @@ SW_EXPORT int simwave_hip_trim_pool(void)
             fail("no default memory pool on the current device");
         int dev = 0;
         hip_check(hipGetDevice(&dev), "hipGetDevice");
-        DeviceArena::drop_blocks(dev, 0, nullptr);
+        sw::drop_blocks<DeviceMemory>(dev, 0, nullptr);
         hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");
         hip_check(hipMemPoolTrimTo(pool, 0), "hipMemPoolTrimTo");
         return 0.0;
