@@ -99,6 +99,9 @@ thread_local double g_timings[8];
 struct Failure {
     std::string msg;
 };
+// ... where the run needs more device memory than there is.
+struct OutOfMemory : Failure {
+};
 
 [[noreturn]] void fail(const char *fmt, ...)
 {
@@ -346,7 +349,14 @@ struct DeviceMemory {
     static void *evict(int device, size_t limit) { return simwave_hip_block_evict(device, limit); }
     [[noreturn]] static void out_of_memory(size_t bytes)
     {
-        fail("hipMallocAsync: out of memory (%zu bytes)", bytes);
+        throw OutOfMemory{{"hipMallocAsync: out of memory (a request of " +
+                           std::to_string(bytes) + " bytes)"}};
+    }
+    // most bytes that one run may take (SIMWAVE_HIP_RUN_MB; 0: no bound)
+    static size_t limit()
+    {
+        const char *v = getenv("SIMWAVE_HIP_RUN_MB");
+        return v && *v ? (size_t)std::max(0, atoi(v)) << 20 : 0;
     }
     [[noreturn]] static void region_full(size_t bytes, size_t cap, size_t used)
     {
@@ -374,6 +384,22 @@ void keep_pool_memory()
             (void)hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &thr);
         }
     });
+}
+
+// Runs f(false); where that finds too little device memory, f(true), whose
+// prepare() leaves out the tiled kernel and its packed coefficients (one value
+// per point more than the z-marching kernel's arrays, with variable density
+// four to six more): a grid that fits without them still runs.
+template <typename F>
+auto within_memory(F f) -> decltype(f(false))
+{
+    try {
+        return f(false);
+    } catch (const OutOfMemory &) {
+        if (SW_DIM == 2)
+            throw;
+    }
+    return f(true);
 }
 
 // Everything the time loop needs on the device, independent of the slots.
@@ -496,9 +522,9 @@ void rho_diff(Prepared &pr, DeviceArena &arena, hipStream_t st)
 
 // Uploads the run constants (the arguments passed validate()).
 // `dev_models` tells whether vel/rho/damp are device pointers (device
-// entry) or host pointers.
+// entry) or host pointers; `lean` leaves out the tiled kernel (within_memory).
 Prepared prepare(const Args &a, bool dev_models, unsigned flags,
-                 DeviceArena &arena, hipStream_t st)
+                 DeviceArena &arena, hipStream_t st, bool lean = false)
 {
     Prepared pr;
     const int r = (int)(a.space_order / 2);
@@ -619,7 +645,7 @@ Prepared prepare(const Args &a, bool dev_models, unsigned flags,
     if (fused && !env_flag("SIMWAVE_HIP_UNTILED")) {
         const char *tile = getenv("SIMWAVE_HIP_TILE");
         const bool want_tile = tile && *tile;
-        if (!env_flag("SIMWAVE_HIP_ZMARCH") && (want_tile || !prefer_zmarch(pr)))
+        if (!lean && !env_flag("SIMWAVE_HIP_ZMARCH") && (want_tile || !prefer_zmarch(pr)))
             setup_tiling(pr, arena, st);
         if (!pr.tiled) {
             pr.zmarch = true;
@@ -638,7 +664,7 @@ Prepared prepare(const Args &a, bool dev_models, unsigned flags,
     // fewer than 2048 blocks (448^3 so8: 854 us at 16 planes, 894 at 8;
     // 176^3 so8: 65 us at 4 planes, 71 at 16)
     const bool oblong = a.nx != a.ny;
-    if (fused && prefer_tiled_vd(pr, oblong, arena))
+    if (fused && !lean && prefer_tiled_vd(pr, oblong, arena))
         setup_tiling(pr, arena, st);
     if (oblong && !pr.tiled)
         fused = pr.fused = false;
@@ -1784,7 +1810,7 @@ std::vector<unsigned long long> frame_indices(const Params &P)
 // A slot is downloaded after its last use through SlotDownloader, so the
 // transfers overlap the time loop; its device buffer is reused only after
 // its download has fired.
-double run_host(const Args &a)
+double run_host(const Args &a, bool lean)
 {
     const double t0 = now_s();
     for (double &t : g_timings)
@@ -1834,7 +1860,7 @@ double run_host(const Args &a)
     double t_prep = 0, t_loop = 0, t_down = 0;
     {
         DeviceArena arena(st);
-        Prepared pr = prepare(a, false, 0, arena, st);
+        Prepared pr = prepare(a, false, 0, arena, st, lean);
         const size_t npts = (size_t)pr.npts;
         const size_t slot_bytes = npts * sizeof(real_t);
 
@@ -1846,17 +1872,16 @@ double run_host(const Args &a)
         std::vector<real_t *> pool;
         std::map<real_t *, hipEvent_t> free_after;   // buffer -> download done
         auto acquire = [&]() -> real_t * {
-            if (!pool.empty()) {
-                real_t *p = pool.back();
-                pool.pop_back();
-                auto it = free_after.find(p);
-                if (it != free_after.end()) {
-                    hip_check(hipStreamWaitEvent(st, it->second, 0), "hipStreamWaitEvent");
-                    free_after.erase(it);
-                }
-                return p;
+            if (pool.empty())
+                return arena.alloc<real_t>(npts);
+            real_t *p = pool.back();
+            pool.pop_back();
+            auto it = free_after.find(p);
+            if (it != free_after.end()) {
+                hip_check(hipStreamWaitEvent(st, it->second, 0), "hipStreamWaitEvent");
+                free_after.erase(it);
             }
-            return arena.alloc<real_t>(npts);
+            return p;
         };
         // bucket slots by the step that uploads / downloads them
         std::vector<std::vector<size_t>> up_at(plan.size()), down_at(plan.size());
@@ -1868,6 +1893,18 @@ double run_host(const Args &a)
             down_at[last[sl]].push_back(sl);
             const StepSlots &s = plan[first[sl]];
             any_frame |= s.next == sl && s.prev != sl && s.cur != sl;
+        }
+        // as many buffers as slots are resident at once, before the first
+        // download: a run that finds too little memory has written nothing
+        {
+            size_t resident = 0, most = 0;
+            for (size_t idx = 0; idx < plan.size(); idx++) {
+                resident += up_at[idx].size();
+                most = std::max(most, resident);
+                resident -= down_at[idx].size();
+            }
+            while (pool.size() < most)
+                pool.push_back(arena.alloc<real_t>(npts));
         }
         // halo frame: indices on the device, packed values staged pinned
         std::vector<unsigned long long> fidx;
@@ -2270,7 +2307,7 @@ void setup_persist(Plan &p)
 }
 #endif
 
-Plan *make_plan(const Args &a, hipStream_t st, unsigned flags)
+Plan *make_plan(const Args &a, hipStream_t st, unsigned flags, bool lean)
 {
     validate(a);
     keep_pool_memory();
@@ -2287,7 +2324,7 @@ Plan *make_plan(const Args &a, hipStream_t st, unsigned flags)
             fail("slot %zu used by step %zu is outside the %zu snapshots", m,
                  a.n0 + idx, a.num_snapshots);
     }
-    p->pr = prepare(a, true, flags, p->arena, st);
+    p->pr = prepare(a, true, flags, p->arena, st, lean);
     if ((flags & kFlagGraph) && !(flags & (kFlagOverlapReceivers | kFlagTimeSteps)) &&
         p->slots.size() >= kGraphSteps && periodic_slots(p->slots))
         capture_graph(*p);
@@ -2298,6 +2335,11 @@ Plan *make_plan(const Args &a, hipStream_t st, unsigned flags)
     hip_check(hipEventCreateWithFlags(&p->last, hipEventDisableTiming), "hipEventCreate");
     hip_check(hipEventRecord(p->last, st), "hipEventRecord");
     return p.release();
+}
+
+Plan *make_plan(const Args &a, hipStream_t st, unsigned flags)
+{
+    return within_memory([&](bool lean) { return make_plan(a, st, flags, lean); });
 }
 
 // Enqueues the next `count` steps of the plan on `st` (after all earlier
@@ -2730,14 +2772,14 @@ RecGather build_rec_gather(const Args &a, const Prepared &pr, DeviceArena &arena
 }
 
 double run_adjoint(const Args &a, const real_t *rec_adj, double *grad, real_t *gw, size_t K,
-                   hipStream_t st, unsigned flags)
+                   hipStream_t st, unsigned flags, bool lean)
 {
     const double t0 = now_s();
     for (double &t : g_timings)
         t = 0.0;
     validate(a);
 #if SW_VD
-    (void)rec_adj; (void)grad; (void)gw; (void)K; (void)st; (void)flags;
+    (void)rec_adj; (void)grad; (void)gw; (void)K; (void)st; (void)flags; (void)lean;
     fail("the adjoint covers constant density only");
     return -1.0;
 #else
@@ -2782,7 +2824,7 @@ double run_adjoint(const Args &a, const real_t *rec_adj, double *grad, real_t *g
     } trim;
     DeviceArena arena(st);
     arena.keep_blocks();
-    Prepared pr = prepare(a, true, 0u, arena, st);
+    Prepared pr = prepare(a, true, 0u, arena, st, lean);
     if (pr.halo_sources)
         fail("the adjoint needs every source box inside the interior");
     const RecGather rg = build_rec_gather(a, pr, arena, st);
@@ -3089,12 +3131,18 @@ static Args fill_args(SW_FORWARD_PARAMS)
 // runtime-compiled wave.c (middleware.py:26-51).
 SW_EXPORT double forward(SW_FORWARD_PARAMS)
 {
-    return guarded([&] { return run_host(fill_args(SW_FORWARD_ARGS)); });
+    return guarded([&] {
+        const Args a = fill_args(SW_FORWARD_ARGS);
+        return within_memory([&](bool lean) { return run_host(a, lean); });
+    });
 }
 
 SW_EXPORT double SW_SUFFIX(simwave_hip_forward_)(SW_FORWARD_PARAMS)
 {
-    return guarded([&] { return run_host(fill_args(SW_FORWARD_ARGS)); });
+    return guarded([&] {
+        const Args a = fill_args(SW_FORWARD_ARGS);
+        return within_memory([&](bool lean) { return run_host(a, lean); });
+    });
 }
 
 SW_EXPORT double SW_SUFFIX(simwave_hip_forward_device_)(SW_FORWARD_PARAMS, void *stream,
@@ -3210,8 +3258,11 @@ SW_EXPORT double SW_SUFFIX(simwave_hip_gradient_)(SW_FORWARD_PARAMS, const real_
                                                  unsigned flags)
 {
     return guarded([&] {
-        return run_adjoint(fill_args(SW_FORWARD_ARGS), rec_adjoint, grad_velocity,
-                           grad_wavelet, checkpoint_every, (hipStream_t)stream, flags);
+        const Args a = fill_args(SW_FORWARD_ARGS);
+        return within_memory([&](bool lean) {
+            return run_adjoint(a, rec_adjoint, grad_velocity, grad_wavelet, checkpoint_every,
+                               (hipStream_t)stream, flags, lean);
+        });
     });
 }
 

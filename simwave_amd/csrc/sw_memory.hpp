@@ -43,6 +43,9 @@ struct Arena {
     };
     int keep_device = -1;
     std::vector<Block> blocks;
+    // bytes requested so far, and the most of them that the run may (0: any)
+    size_t requested = 0;
+    const size_t limit = Api::limit();
 
     explicit Arena(Stream s) : stream(s) {}
     Arena(Stream s, void *region, size_t bytes)
@@ -110,6 +113,9 @@ struct Arena {
             used += whole;
             return static_cast<T *>(p);
         }
+        requested += bytes;
+        if (limit && requested > limit)
+            Api::out_of_memory(bytes);
         if (keep_device >= 0 && bytes >= kKeepMin)
             return static_cast<T *>(alloc_block(bytes));
         ptrs.reserve(ptrs.size() + 1);

@@ -35,6 +35,7 @@ static size_t total(const std::map<void *, size_t> &m)
     return s;
 }
 struct Full {};
+static size_t bound = 0;
 struct Stub {
     typedef int stream;
     static int device() { return 0; }
@@ -93,6 +94,7 @@ struct Stub {
         return p;
     }
     [[noreturn]] static void out_of_memory(size_t) { throw Full{}; }
+    static size_t limit() { return bound; }
     [[noreturn]] static void region_full(size_t, size_t, size_t) { throw Full{}; }
 };
 typedef sw::Arena<Stub> Arena;
@@ -149,6 +151,11 @@ int main()
     bool full = false;
     try { Arena a(0); a.alloc<char>(10 * MB); a.alloc<char>(60 * MB); } catch (Full) { full = true; }
     CHECK(full && live.empty() && total(kept) == 0);
+    bound = 4 * MB;                          // a bound on one run
+    full = false;
+    try { Arena a(0); a.alloc<char>(3 * MB); a.alloc<char>(2 * MB); } catch (Full) { full = true; }
+    CHECK(full && live.empty());
+    bound = 0;
     char region[1024];
     Arena r(0, region, sizeof region);       // a caller's region
     CHECK(r.alloc<char>(1) == region && r.alloc<float>(64) == (float *)(region + 256));
