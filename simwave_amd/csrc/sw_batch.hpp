@@ -33,9 +33,11 @@ struct BatchShot {
 constexpr int kMaxBatch = 48;
 
 #if SW_DIM == 3
-constexpr int kBatchLines = kZLines, kRecPerBatch = kRecPerZ, kRecChunkBatch = kRecChunkZ;
+constexpr int kBatchLines = kZLines, kRecPerBatch = kRecPerZ;
+typedef RecZ RecBatch;
 #else
-constexpr int kBatchLines = 4, kRecPerBatch = sizeof(real_t) == 4 ? 16 : 8, kRecChunkBatch = 128;
+constexpr int kBatchLines = 4, kRecPerBatch = sizeof(real_t) == 4 ? 16 : 8;
+typedef RecShared<kRecPerBatch, 128> RecBatch;
 #endif
 
 // Arguments of one batched launch (by value): the shots, their step numbers
@@ -62,7 +64,7 @@ __device__ __forceinline__ int batch_shot(const BatchArgs &A, int b)
 
 template <int R>
 #if SW_DIM == 3
-__global__ void __launch_bounds__(64 * kZLines)
+__global__ void __launch_bounds__(64 * kZLines, z_waves(R))
 k_step3d_z_batch(BatchArgs A)
 #else
 __global__ void __launch_bounds__(kZ2Block)
@@ -70,7 +72,7 @@ k_step2d_z_batch(BatchArgs A)
 #endif
 {
     constexpr int NT = SW_DIM == 3 ? 64 * kBatchLines : 256;
-    __shared__ RecShared<kRecPerBatch, kRecChunkBatch> sh;
+    __shared__ RecBatch sh;
     const int s = batch_shot(A, blockIdx.x);
     const BatchShot *__restrict__ b = A.shot[s];
     const Params P = b->P;
@@ -80,9 +82,9 @@ k_step2d_z_batch(BatchArgs A)
     real_t *u = b->u;
     const real_t *uc = u + (long long)(n % 3) * np;
     if (local < b->nrb) {
-        receivers_block<NT>(P, sh, uc, b->rbox, b->rw, b->nrec,
-                            b->rec + (long long)(n - 1) * b->nrec, local,
-                            SW_DIM == 3 ? threadIdx.y * 64 + threadIdx.x : threadIdx.x);
+        receivers_beside<NT, R>(P, sh, uc, b->rbox, b->rw, b->nrec,
+                                b->rec + (long long)(n - 1) * b->nrec, local,
+                                SW_DIM == 3 ? threadIdx.y * 64 + threadIdx.x : threadIdx.x);
         return;
     }
     local -= b->nrb;

@@ -926,7 +926,8 @@ void tiled_launch(const Prepared &pr, const real_t *uc, const real_t *up, real_t
     A.nsrc = P.nsrc;
     A.sbox = P.sbox;
     A.T = pr.tiling;
-    rec.nrb = (rec.nrec + sw::kRecPerWave * NW - 1) / (sw::kRecPerWave * NW);
+    constexpr int per_block = sw::RecTile<sw::TileShape<R, WR, RPT, NW, V>, R, NW>::RPB;
+    rec.nrb = (rec.nrec + per_block - 1) / per_block;
     rec.nrb = (rec.nrb + 7) / 8 * 8;
     // the gather's blocks, in groups of 8, spread over the first three quarters
     // of the launch: all at the front they delay the step (472^3: 57.6 ms per

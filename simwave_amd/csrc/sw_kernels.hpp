@@ -389,29 +389,31 @@ __device__ __forceinline__ void store_with_bc(const Params &P, real_t *un,
 // writes of a wave's receivers do not collide.  16384 receivers of 9^3
 // points at 472^3: 28 us alone per step, 56 before (single loads, the
 // chain waiting for every LDS read).
-constexpr int kRecWeights = 64;           // weights kept in LDS per receiver
+// Axis weights kept in LDS per receiver (WC): a wider box reads them from
+// memory.  The step launches' gathers keep 32, the default window's three
+// axes taking 27, for the sake of the step's occupancy.
+constexpr int kRecWeights = 64, kRecWeightsStep = 32;
 
-template <int RPB, int CH>
+template <int RPB, int CH, int WC = kRecWeights>
 struct RecShared {
     static constexpr int ROW = CH + 64 / (int)sizeof(real_t);
     static_assert(CH * sizeof(real_t) % 256 == 0, "LDS row layout");
     alignas(16) real_t prod[RPB][ROW];
-    real_t wts[RPB][kRecWeights + 1];
+    real_t wts[RPB][WC + 1];
     int counts[RPB], nweights[RPB];
 };
 
-// Receivers bx*RPB .. bx*RPB+RPB-1 of one shot; tid: the thread in the block.
-template <int NT, int RPB, int CH>
-__device__ __forceinline__ void receivers_block(const Params &P, RecShared<RPB, CH> &sh,
+// Receivers bx*RPB .. bx*RPB+RPB-1 of one shot; tid: the thread in the block;
+// NB: box values in flight per thread; GRP: products per step of the chain.
+template <int NT, int NB = 8, int GRP = 16, int RPB, int CH, int WC>
+__device__ __forceinline__ void receivers_block(const Params &P, RecShared<RPB, CH, WC> &sh,
                                                 const real_t *__restrict__ uc,
                                                 const Box *__restrict__ rbox,
                                                 const real_t *__restrict__ rw, int nrec,
                                                 real_t *__restrict__ out, int bx, int tid)
 {
     constexpr int STEP = NT / RPB;        // threads of one receiver
-    constexpr int NB = 8;                 // box values in flight per thread
-    constexpr int GRP = 16;               // products per step of the chain
-    constexpr int WCAP = kRecWeights;
+    constexpr int WCAP = WC;
     static_assert(CH % GRP == 0 && RPB <= 64 && NT % RPB == 0, "block layout");
     typedef real_t vec16 __attribute__((ext_vector_type(16 / sizeof(real_t))));
     constexpr int V = 16 / (int)sizeof(real_t);
@@ -531,6 +533,22 @@ __device__ __forceinline__ void receivers_block(const Params &P, RecShared<RPB, 
     }
     if (tid < RPB && r0 + tid < nrec)
         out[r0 + tid] = acc;
+}
+
+// The gather beside a step in one launch.  In float64, beside 3D steps of few
+// registers, half as many box values and products are in flight: the whole
+// number takes 99 registers, the z-marching step of radius 1 59.
+constexpr bool rec_light(int R) { return SW_DIM == 3 && sizeof(real_t) == 8 && R <= 3; }
+
+template <int NT, int R, typename Shared>
+__device__ __forceinline__ void receivers_beside(const Params &P, Shared &sh,
+                                                 const real_t *__restrict__ uc,
+                                                 const Box *__restrict__ rbox,
+                                                 const real_t *__restrict__ rw, int nrec,
+                                                 real_t *__restrict__ out, int bx, int tid)
+{
+    receivers_block<NT, rec_light(R) ? 4 : 8, rec_light(R) ? 8 : 16>(P, sh, uc, rbox, rw, nrec,
+                                                                     out, bx, tid);
 }
 
 // ------------------------------------------------ fused step, 3D
@@ -847,21 +865,34 @@ struct RecArgs {
 };
 
 // The z-marching kernels' gather: 16 receivers per block, rounds of 256 (128
-// in float64) products, 17 KB of LDS, which leaves the step's occupancy.
+// in float64) products, 20 KB of LDS (22 KB): 8 (7) blocks per CU, as many as
+// the step's registers allow.
 constexpr int kRecPerZ = 16;
 constexpr int kRecChunkZ = sizeof(real_t) == 4 ? 256 : 128;
+typedef RecShared<kRecPerZ, kRecChunkZ, kRecWeightsStep> RecZ;
+
+// Wavefronts per SIMD asked of the compiler for the radii where it would give
+// the two paths of a launch together a few registers more than the step alone
+// and one wavefront less (116^3 variable density so8 with 4096 receivers, 100
+// steps: 4.5 -> 3.5 ms); elsewhere its own choice is as fast or faster.
+constexpr int z_waves(int R)
+{
+    if (sizeof(real_t) == 8)
+        return SW_VD ? 1 : R == 1 ? 7 : R == 2 ? 6 : R == 3 ? 5 : 1;
+    return SW_VD ? (R == 4 || R == 8 ? 4 : 1) : (R >= 9 ? 4 : 1);
+}
 
 template <int R>
-__global__ void __launch_bounds__(64 * kZLines)
+__global__ void __launch_bounds__(64 * kZLines, z_waves(R))
 k_step3d_z(Params P, LapDiv D, const real_t *__restrict__ uc, const real_t *__restrict__ up,
            real_t *__restrict__ un, int n, int zlen, int gx, int gy, RecArgs rec)
 {
-    __shared__ RecShared<kRecPerZ, kRecChunkZ> sh;
+    __shared__ RecZ sh;
     if ((int)blockIdx.x < rec.nrb) {
         if (P.nbase)
             rec.out += (long long)(*P.nbase) * rec.nrec;
-        receivers_block<64 * kZLines>(P, sh, uc, rec.rbox, rec.rw, rec.nrec, rec.out, blockIdx.x,
-                                      threadIdx.y * 64 + threadIdx.x);
+        receivers_beside<64 * kZLines, R>(P, sh, uc, rec.rbox, rec.rw, rec.nrec, rec.out,
+                                          blockIdx.x, threadIdx.y * 64 + threadIdx.x);
         return;
     }
     const int s = blockIdx.x - rec.nrb, t = s / gx;

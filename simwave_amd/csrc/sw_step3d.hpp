@@ -325,16 +325,6 @@ struct StepArgs {
     Tiling T;
 };
 
-// Receivers per wavefront of the gather in the step launch, and products per
-// round (9 KB of LDS, no more than the step's tile).  A gathering wavefront
-// takes a step wavefront's registers, so it serves several receivers (100
-// steps of 472^3 with 16384 receivers: 59.1 ms at 2 per wavefront, 58.2 at 4,
-// 57.6 at 8).
-constexpr int kRecPerWave = 8;
-constexpr int kRecChunkVec = sizeof(real_t) == 4 ? 256 : 128;
-template <int NW>
-using RecVec = RecShared<kRecPerWave * NW, kRecChunkVec>;
-
 // Whether x is a subnormal number.
 __device__ __forceinline__ bool subnormal(float x)
 {
@@ -359,6 +349,29 @@ struct TileShape {
     static constexpr int NC = LP / kVec16;             // 16-byte chunks per lane and value
     static_assert(LP % kVec16 == 0, "a lane's packed values fill whole 16-byte chunks");
     static constexpr int NA(int rho) { return rho ? 5 : 1; }   // packed values per point
+    static constexpr int PLANE = H * LS + 64 * NW * V;         // LDS plane and dump slots
+};
+
+// The gather in a tile's step launch: receivers per block, products per round.
+// A gathering wavefront takes a step wavefront's registers, so it serves
+// several receivers (100 steps of 472^3 with 16384 receivers: 59.1 ms at 2 per
+// wavefront, 58.2 at 4, 57.6 at 8); 4 where it has half the loads in flight
+// (rec_light), which leaves a box as many waits for memory.  Its LDS is every
+// block's, so it must leave the wavefronts per SIMD that the step's registers
+// allow (kTileWaves).  With 8 receivers and 64 weights each for every tile (11
+// and 13 KB of LDS, where a tile takes from 4 KB on) the float64 tiles of
+// radius 1 to 3 ran 3 wavefronts per SIMD where their registers allow 7, 5 and
+// 4 (100 steps of 180^3 with 4096 receivers: so2 7.0 -> 6.0 ms, so4 6.6 -> 5.5, so6 7.2 -> 6.0).
+template <int R>
+constexpr int kTileWaves = kVec16 == 4 ? 4 : R == 1 ? 7 : R == 2 ? 5 : R == 3 ? 4 : 3;
+template <typename S, int R, int NW>
+struct RecTile {
+    static constexpr int RPB = NW * (rec_light(R) ? 4 : 8);
+    typedef RecShared<RPB, sizeof(real_t) == 4 ? 256 : 128, kRecWeightsStep> Shared;
+    static constexpr size_t lds_step = 2 * S::PLANE * sizeof(real_t);
+    static constexpr size_t lds = sizeof(Shared) > lds_step ? sizeof(Shared) : lds_step;
+    static_assert(lds == lds_step || lds <= (size_t)40960 * NW / kTileWaves<R>,
+                  "the gather's LDS takes the step's wavefronts");
 };
 
 // D64 (float32 only): the Laplacian quotients sum/h2 as RN(sum * RN(1/h2)),
@@ -388,9 +401,9 @@ k_step3d_vec(StepArgs A, const Params *__restrict__ Pd, int n)
     // two plane buffers, each followed by one dump slot per thread that
     // takes the halo writes of lanes without a halo vector, so that every
     // lane issues the same LDS stores (no branches around them)
-    constexpr int DUMP = H * LS, PLANE = H * LS + NT * V;
-    constexpr size_t lds_step = 2 * PLANE * esz, lds_rec = sizeof(RecVec<NW>);
-    __shared__ __align__(16) unsigned char smem[lds_step > lds_rec ? lds_step : lds_rec];
+    constexpr int DUMP = H * LS, PLANE = S::PLANE;
+    typedef RecTile<S, R, NW> G;
+    __shared__ __align__(16) unsigned char smem[G::lds];
     real_t *const lds = (real_t *)smem;
 
     const int lane = threadIdx.x, w = threadIdx.y;
@@ -404,8 +417,8 @@ k_step3d_vec(StepArgs A, const Params *__restrict__ Pd, int n)
             real_t *out = A.rec.out;
             if (Pd->nbase)
                 out += (long long)(*Pd->nbase) * A.rec.nrec;
-            receivers_block<NT>(*Pd, *(RecVec<NW> *)smem, A.uc, A.rec.rbox, A.rec.rw,
-                                     A.rec.nrec, out, rg * 8 + (bid & 7), tid);
+            receivers_beside<NT, R>(*Pd, *(typename G::Shared *)smem, A.uc, A.rec.rbox, A.rec.rw,
+                                    A.rec.nrec, out, rg * 8 + (bid & 7), tid);
             return;
         }
         bid -= 8 * min(ng, rg + 1);
