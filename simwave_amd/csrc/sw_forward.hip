@@ -409,6 +409,7 @@ struct Prepared {
     const real_t *rw = nullptr;
     bool fused = false;
     bool halo_sources = false;   // some source box reaches the halo
+    int src_z0 = 0, src_z1 = 0;  // z planes of all source boxes
     int r = 0;
     long long npts = 0;
 #if SW_DIM == 3
@@ -430,7 +431,8 @@ struct Prepared {
 };
 
 #if SW_DIM == 3
-void setup_tiling(Prepared &pr, DeviceArena &arena, hipStream_t st);
+void setup_tiling(Prepared &pr, DeviceArena &arena, hipStream_t st,
+                  const sw::Models *M = nullptr);
 bool prefer_zmarch(const Prepared &pr);
 bool prefer_tiled_vd(const Prepared &pr, bool oblong, const DeviceArena &arena);
 void set_lap_div(Prepared &pr);
@@ -557,22 +559,6 @@ Prepared prepare(const Args &a, bool dev_models, unsigned flags,
         P.c1[m] = SW_VD ? a.c1[m] : (real_t)0;
     }
 
-    // per-point coefficients: upload v and damp into the q/e buffers and
-    // convert in place (k_prepare reads a point before writing it)
-    real_t *q = arena.alloc<real_t>(npts);
-    real_t *e = arena.alloc<real_t>(npts);
-    const hipMemcpyKind mk = dev_models ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-    hip_check(hipMemcpyAsync(q, a.vel, npts * sizeof(real_t), mk, st), "copy velocity");
-    hip_check(hipMemcpyAsync(e, a.damp, npts * sizeof(real_t), mk, st), "copy damp");
-    {
-        const real_t dt = a.dt, dt2 = a.dt * a.dt;
-        const int blocks = (int)std::min<long long>((npts + 255) / 256, 8192);
-        hipLaunchKernelGGL(sw::k_prepare, dim3(blocks), dim3(256), 0, st, q, e, q, e,
-                           npts, dt, dt2);
-        hip_check(hipGetLastError(), "k_prepare launch");
-    }
-    P.q = q;
-    P.e = e;
 #if SW_VD
     if (dev_models) {
         P.rho = a.rho;
@@ -613,6 +599,9 @@ Prepared prepare(const Args &a, bool dev_models, unsigned flags,
             for (int d = 0; d < SW_DIM; d++)
                 if (b.lo[d] < r || b.hi[d] >= (int)dims[d] - r)
                     pr.halo_sources = true;
+            const bool first = pr.src_z1 == 0;
+            pr.src_z0 = first ? b.lo[0] : std::min(pr.src_z0, b.lo[0]);
+            pr.src_z1 = std::max(pr.src_z1, b.hi[0] + 1);
         }
     }
     if (a.nrec) {
@@ -627,6 +616,23 @@ Prepared prepare(const Args &a, bool dev_models, unsigned flags,
         pr.rw = d_rw;
     }
 
+    // per-point coefficients: upload v and damp into the q/e buffers and
+    // convert in place (k_prepare reads a point before writing it)
+    auto coefficients = [&] {
+        real_t *q = arena.alloc<real_t>(npts);
+        real_t *e = arena.alloc<real_t>(npts);
+        const hipMemcpyKind mk = dev_models ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
+        hip_check(hipMemcpyAsync(q, a.vel, npts * sizeof(real_t), mk, st), "copy velocity");
+        hip_check(hipMemcpyAsync(e, a.damp, npts * sizeof(real_t), mk, st), "copy damp");
+        const real_t dt = a.dt, dt2 = a.dt * a.dt;
+        const int blocks = (int)std::min<long long>((npts + 255) / 256, 8192);
+        hipLaunchKernelGGL(sw::k_prepare, dim3(blocks), dim3(256), 0, st, q, e, q, e,
+                           npts, dt, dt2);
+        hip_check(hipGetLastError(), "k_prepare launch");
+        P.q = q;
+        P.e = e;
+    };
+
     // fused-kernel preconditions: interior of every axis at least r+1 thick
     // (Neumann mirrors read interior points only), few sources, and for 3D
     // variable density the middle-axis quirk stride nx equal to ny.
@@ -637,7 +643,12 @@ Prepared prepare(const Args &a, bool dev_models, unsigned flags,
     if (a.nsrc > (size_t)kMaxFusedSources)
         fused = false;
     pr.fused = fused;
+    // (the tiled kernel does without q and e in a caller-owned arena)
+    const bool scratch = SW_DIM == 3 && !SW_VD && arena.base && fused;
+    if (!scratch)
+        coefficients();
 #if SW_DIM == 3 && !SW_VD
+    const sw::Models models{a.vel, a.damp, a.dt, a.dt * a.dt};
     // the z-marching one-point-per-thread kernel where it is the faster one
     // (prefer_zmarch), when asked for, or where the tiled kernel's 32-bit
     // buffer offsets do not fit; the tiled kernel otherwise or when a tile
@@ -646,13 +657,15 @@ Prepared prepare(const Args &a, bool dev_models, unsigned flags,
         const char *tile = getenv("SIMWAVE_HIP_TILE");
         const bool want_tile = tile && *tile;
         if (!lean && !env_flag("SIMWAVE_HIP_ZMARCH") && (want_tile || !prefer_zmarch(pr)))
-            setup_tiling(pr, arena, st);
+            setup_tiling(pr, arena, st, scratch ? &models : nullptr);
         if (!pr.tiled) {
             pr.zmarch = true;
             pr.zmarch_zlen = std::max(1, std::min(env_int("SIMWAVE_HIP_ZLEN", 8), 256));
             set_lap_div(pr);
         }
     }
+    if (scratch && !pr.tiled)
+        coefficients();
 #elif SW_DIM == 3
     // variable density: the tiled kernel where it is the faster one
     // (prefer_tiled_vd) or when asked for (SIMWAVE_HIP_TILE); the z-marching
@@ -1041,9 +1054,15 @@ TiledKernel tiled_kernel(int R, int v)
 // Chooses the tile grid and launch order and marks the tile planes that
 // hold damping.  Leaves pr.tiled false when the grid does not fit the
 // kernel's 32-bit buffer offsets.
-void setup_tiling(Prepared &pr, DeviceArena &arena, hipStream_t st)
+// Tile geometry, damping mask and packed coefficients; leaves pr.tiled false
+// where the kernel does not fit.  M: the models on the device, for a
+// caller-owned arena, which has no room for q and e of every point beside the
+// packed values: those of the source boxes' planes take their place (104 x 120
+// x 140 so16 in float64: 31 us per step, the z-marching kernel 59; 150 x 161 x
+// 183 so12 in float32 36 and 40).
+void setup_tiling(Prepared &pr, DeviceArena &arena, hipStream_t st, const sw::Models *M)
 {
-    const Params &P = pr.P;
+    Params &P = pr.P;
     const int R = pr.r;
     // float32 Laplacian quotients as float64 products with RN(1/h^2) where
     // that gives the IEEE quotient for every numerator, or for all but
@@ -1089,12 +1108,23 @@ void setup_tiling(Prepared &pr, DeviceArena &arena, hipStream_t st)
     if (blocks >= (1ll << 31))
         return;
     T.nwords = P.nz / 32 + 3;
-    // the packed coefficients; a caller-owned arena that cannot take them
-    // leaves the run to the other kernels
     const size_t tile_points = (size_t)T.ncols * Iz * T.ty * T.txr;
-    if (arena.base && tile_points * (SW_VD ? 6 : 2) * sizeof(real_t) + kPackSlack >
-                          arena.cap - arena.used)
-        return;
+    if (M) {
+        const int planes = pr.src_z1 - pr.src_z0;
+        const size_t n = (size_t)planes * (size_t)P.sz;
+        if ((tile_points + n) * 2 * sizeof(real_t) + kPackSlack > arena.cap - arena.used)
+            return;
+        if (n) {
+            real_t *q = arena.alloc<real_t>(n), *e = arena.alloc<real_t>(n);
+            const long long p0 = (long long)pr.src_z0 * P.sz;
+            hipLaunchKernelGGL(sw::k_prepare, dim3((unsigned)std::min<size_t>((n + 255) / 256, 8192)),
+                               dim3(256), 0, st, M->vel + p0, M->damp + p0, q, e, (long long)n,
+                               M->dt, M->dt2);
+            hip_check(hipGetLastError(), "k_prepare launch");
+            P.q = q - p0;
+            P.e = e - p0;
+        }
+    }
     const long long words = (long long)T.ncols * T.nwords + 1;   // + den_bad
     unsigned *mask = arena.alloc<unsigned>((size_t)words);
     {
@@ -1103,9 +1133,9 @@ void setup_tiling(Prepared &pr, DeviceArena &arena, hipStream_t st)
                            dim3(256), 0, st, mask, words);
     }
     T.dmask = mask;
-    hipLaunchKernelGGL(sw::k_damp_flags, dim3(T.ncols, P.nz), dim3(256), 0, st, P.e, P.nz,
-                       P.nx, P.ny, R, T.gk, T.ty, T.txr, T.nwords, mask,
-                       mask + words - 1);
+    hipLaunchKernelGGL(M ? sw::k_damp_flags<true> : sw::k_damp_flags<false>,
+                       dim3(T.ncols, P.nz), dim3(256), 0, st, P, M ? *M : sw::Models{}, P.nz,
+                       P.nx, P.ny, R, T.gk, T.ty, T.txr, T.nwords, mask, mask + words - 1);
     hip_check(hipGetLastError(), "k_damp_flags launch");
     Params *Pd = arena.alloc<Params>(1);
     hip_check(hipMemcpyAsync(Pd, &P, sizeof(Params), hipMemcpyHostToDevice, st),
@@ -1113,8 +1143,9 @@ void setup_tiling(Prepared &pr, DeviceArena &arena, hipStream_t st)
     pr.Pd = Pd;
     real_t *pk = arena.alloc<real_t>(tile_points * (SW_VD ? 5 : 1));
     real_t *pe = arena.alloc<real_t>(tile_points);
-    hipLaunchKernelGGL(sw::k_pack_tiles, dim3(T.ncols, Iz), dim3(256), 0, st, P, R, K.pack, T.gk,
-                       T.ty, T.txr, T.ncols, SW_VD, pk, pe);
+    hipLaunchKernelGGL(M ? sw::k_pack_tiles<true> : sw::k_pack_tiles<false>, dim3(T.ncols, Iz),
+                       dim3(256), 0, st, P, M ? *M : sw::Models{}, R, K.pack, T.gk, T.ty, T.txr,
+                       T.ncols, SW_VD, pk, pe);
     hip_check(hipGetLastError(), "k_pack_tiles launch");
     pr.pk = pk;
     pr.pe = pe;
@@ -2511,8 +2542,11 @@ double run_device_noalloc(const Args &a, hipStream_t st, unsigned flags)
             fail("slot %zu used by step %zu is outside the %zu snapshots", m,
                  a.n0 + idx, a.num_snapshots);
     }
-    // the per-point arrays (q, e and, for the tiled 3D kernel, C) decide
-    // whether the grid fits; the small tables follow them
+    // the per-point arrays decide whether the grid fits, and small tables stand
+    // beside them: q and e, or for the tiled 3D kernel its packed coefficients,
+    // two values per point of whole tiles; three values per point leave room
+    // for the tiles' padding (a grid whose tiles need more takes the
+    // z-marching kernel)
     const size_t npts = a.nz * a.nx * (SW_DIM == 3 ? a.ny : 1);
     // variable density from radius sw::kVdPre on adds the density sums
     const size_t per_point =
@@ -2540,6 +2574,12 @@ double run_device_noalloc(const Args &a, hipStream_t st, unsigned flags)
               swap, no_uploads);
     hip_check(hipStreamSynchronize(st), "time loop");
     g_timings[2] = now_s() - tl0;
+    g_timings[6] = pr.fused ? 1.0 : 0.0;
+#if SW_DIM == 3
+    g_timings[7] = pr.tiled ? 1.0 : pr.zmarch ? 2.0 : 0.0;
+#else
+    g_timings[7] = pr.fused && zmarch_2d(pr.r) ? 2.0 : 0.0;
+#endif
     g_timings[0] = now_s() - t0;
     return g_timings[0];
 }
@@ -2622,8 +2662,9 @@ AdjPlan plan_adjoint(Prepared &pr, DeviceArena &arena, hipStream_t st)
                        dim3((unsigned)std::min<long long>((words + 255) / 256, 4096)), dim3(256),
                        0, st, mask, words);
     T.dmask = mask;
-    hipLaunchKernelGGL(sw::k_damp_flags, dim3(T.ncols, P.nz), dim3(256), 0, st, P.e, P.nz, P.nx,
-                       P.ny, R, T.gk, T.ty, T.txr, T.nwords, mask, mask + words - 1);
+    hipLaunchKernelGGL(sw::k_damp_flags<false>, dim3(T.ncols, P.nz), dim3(256), 0, st, P,
+                       sw::Models{}, P.nz, P.nx, P.ny, R, T.gk, T.ty, T.txr, T.nwords, mask,
+                       mask + words - 1);
     hip_check(hipGetLastError(), "k_damp_flags launch");
 #else
     (void)arena;

@@ -225,6 +225,15 @@ __device__ __forceinline__ real_t add_sources(const Params &P, int n, int i,
 // wave.c:177-181 (per-point terms that do not depend on the time step).
 // Called in place (q aliases vel, e aliases damp): each point is read
 // before it is written, by the same thread.
+__device__ __forceinline__ real_t prepared_s(real_t v)
+{
+    return (real_t)(1.0 / (double)(v * v));
+}
+__device__ __forceinline__ real_t prepared_q(real_t v, real_t dt2) { return dt2 / prepared_s(v); }
+__device__ __forceinline__ real_t prepared_e(real_t v, real_t damp, real_t dt)
+{
+    return damp * dt / (2 * prepared_s(v));
+}
 __global__ void k_prepare(const real_t *vel, const real_t *damp,
                           real_t *q, real_t *e,
                           long long npts, real_t dt, real_t dt2)
@@ -232,9 +241,9 @@ __global__ void k_prepare(const real_t *vel, const real_t *damp,
     for (long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
          p < npts; p += (long long)gridDim.x * blockDim.x) {
         const real_t v = vel[p];
-        const real_t s = (real_t)(1.0 / (double)(v * v));
-        q[p] = dt2 / s;
-        e[p] = damp[p] * dt / (2 * s);
+        const real_t d = damp[p];
+        q[p] = prepared_q(v, dt2);
+        e[p] = prepared_e(v, d, dt);
     }
 }
 

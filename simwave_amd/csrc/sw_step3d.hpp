@@ -60,10 +60,10 @@ struct Tiling {
 };
 
 // Sources restricted to the tile's mask, in index order (the reference's
-// sequential += order, wave.c:208-295).
-__device__ __forceinline__ real_t add_sources_masked(const Params &P, int n, int i,
-                                                     int j, int k, real_t qv,
-                                                     real_t ev, real_t v,
+// sequential += order, wave.c:208-295).  q and e are read inside the source
+// boxes only: the allocation-free entry holds no others.
+__device__ __forceinline__ real_t add_sources_masked(const Params &P, int n, int i, int j, int k,
+                                                     long long p, real_t v,
                                                      unsigned long long mask)
 {
     while (mask) {
@@ -77,15 +77,34 @@ __device__ __forceinline__ real_t add_sources_masked(const Params &P, int n, int
         const real_t amp = wavelet_amp(P, n, s);
         if (amp == (real_t)0)
             continue;
-        v += source_term(qv, ev, box_weight(b, P.sw, i, j, k), amp);
+        v += source_term(P.q[p], P.e[p], box_weight(b, P.sw, i, j, k), amp);
     }
     return v;
 }
 
+// Where the set-up kernels take a point's coefficients q and e from: the arrays
+// of k_prepare, or (RAW) the velocity and damping models, by k_prepare's
+// operations.
+struct Models {
+    const real_t *vel, *damp;
+    real_t dt, dt2;
+};
+template <bool RAW>
+__device__ __forceinline__ real_t point_q(const Params &P, const Models &M, long long p)
+{
+    return RAW ? prepared_q(M.vel[p], M.dt2) : P.q[p];
+}
+template <bool RAW>
+__device__ __forceinline__ real_t point_e(const Params &P, const Models &M, long long p)
+{
+    return RAW ? prepared_e(M.vel[p], M.damp[p], M.dt) : P.e[p];
+}
+
 // Marks tile planes holding a non-zero damping term.  grid (ncols, nz); the
 // mask words must be zeroed beforehand.
+template <bool RAW>
 __global__ void __launch_bounds__(256)
-k_damp_flags(const real_t *__restrict__ e, int nz, int nx, int ny, int R, int gk,
+k_damp_flags(Params P, Models M, int nz, int nx, int ny, int R, int gk,
              int ty, int txr, int nwords, unsigned *__restrict__ mask,
              unsigned *__restrict__ den_bad)
 {
@@ -96,7 +115,7 @@ k_damp_flags(const real_t *__restrict__ e, int nz, int nx, int ny, int R, int gk
     for (int t = threadIdx.x; t < ty * txr; t += blockDim.x) {
         const int k = k0 + t % ty, j = j0 + t / ty;
         if (k < ny && j < nx) {
-            const real_t v = e[((long long)z * nx + j) * ny + k];
+            const real_t v = point_e<RAW>(P, M, ((long long)z * nx + j) * ny + k);
             if (v != (real_t)0) {
                 const double den = fabs((double)(real_t)(1.0 + (double)v));
                 any |= den >= 0x1p-60 && den <= 0x1p60 ? 1 : 3;
@@ -129,8 +148,9 @@ struct PackShape {
 // damping terms in the same order.  Values outside the interior are zero.
 // The sums are formed in the reference's order (vd-3d wave.c:175-186, where
 // the x axis steps by nx elements) from +0.
+template <bool RAW>
 __global__ void __launch_bounds__(256)
-k_pack_tiles(Params P, int R, PackShape S, int gk, int ty, int txr, int ncols, int rho,
+k_pack_tiles(Params P, Models M, int R, PackShape S, int gk, int ty, int txr, int ncols, int rho,
              real_t *__restrict__ pk, real_t *__restrict__ pe)
 {
     const int lp = S.rpt * S.v, nc = lp / kVec16, na = rho ? 5 : 1;
@@ -148,8 +168,8 @@ k_pack_tiles(Params P, int R, PackShape S, int gk, int ty, int txr, int ncols, i
         real_t v[5] = {0, 0, 0, 0, 0}, e = 0;
         if (j < P.nx - R && k < P.ny - R) {
             const long long p = (long long)i * P.sz + (long long)j * P.sx + k;
-            e = P.e[p];
-            v[0] = P.q[p] / (real_t)(1.0 + (double)e);
+            e = point_e<RAW>(P, M, p);
+            v[0] = point_q<RAW>(P, M, p) / (real_t)(1.0 + (double)e);
             if (rho) {
                 const real_t *__restrict__ d = P.rho + p;
                 for (int m = 1; m <= R; m++) {
@@ -912,8 +932,7 @@ k_step3d_vec(StepArgs A, const Params *__restrict__ Pd, int n)
                     const long long p = (long long)i * nx * ny + (long long)j * ny + kk;
                     real_t v = out[q][e];
                     if (smask)
-                        v = add_sources_masked(*Pd, n, i, j, kk, Pd->q[p], Pd->e[p], v,
-                                               smask);
+                        v = add_sources_masked(*Pd, n, i, j, kk, p, v, smask);
                     if (bc_here)
                         store_with_bc(*Pd, A.un, p, i, j, kk, v);
                     else
