@@ -832,12 +832,24 @@ int default_tile(int R, bool div64, long long interior)
 // 4 planes fetch 0.82 GB per step and take 185 us, 12 planes 212 us, 24
 // planes 1.02 GB); large grids and the long prologues of high orders want a
 // few more (472^3: 6 planes 502 us, 4 514; so16 float64 240^3: 12 planes 168,
-// 4 178), small grids fewer, to fill the chip (148^3 variable density so8: 2
-// planes 38.1 us, 4 40.0; 168^3 so16 42.3 and 43.9).
+// 4 178), small grids fewer, to fill the chip: below 1 M interior points 2
+// planes everywhere (56^3 so10 12.8 us, 4 planes 19.8; 53^3 float64 so16 9.9
+// and 13.4), up to 5 M still 2 for float32 up to radius 8 and for constant
+// density in float64 up to radius 3 (150^3 so12 32.1, 4 planes 33.0; 150^3
+// variable density so8 37.3 and 40.7; 142^3 float64 so4 28.2 and 30.4), which
+// the longer prologues of the others lose (2 planes, 4 planes: 160^3 so20 61.4,
+// 57.1; 160^3 variable density so20 135, 127; float64 142^3 so10 49.4, 44.4,
+// 160^3 so8 53.2, 50.4, variable density 142^3 so8 57.0, 53.8, so4 160^3 89.7,
+// 84.5), more so in float64 from radius 8 on (142^3 variable density so16 112,
+// 104, 6 planes 96; 160^3 so20 86.7, 74.8, 72.4).
 int default_tile_zlen(int R, long long interior)
 {
-    if (interior < 5ll * 1000 * 1000)
-        return 2;
+    const long long M = 1000 * 1000;
+    if (interior < 5 * M) {
+        if (interior < M || (kF32 ? R < 9 : !SW_VD && (R < 4 || (R == 4 && interior < 3 * M))))
+            return 2;
+        return !kF32 && R >= 8 && interior >= 3 * M ? 6 : 4;
+    }
     if (SW_VD)
         return kF32 ? (R < 8 ? 4 : 6) : (R < 6 ? 4 : 8);
     if (R == 4)
