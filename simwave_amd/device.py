@@ -43,6 +43,25 @@ def _is_torch_tensor(x):
     return type(x).__module__.split(".")[0] == "torch"
 
 
+def library_bytes(shape, space_order, itemsize, density):
+    """Most bytes of per-point arrays that the library holds for a shot on the
+    extended grid `shape`, whichever kernel it takes.  2D: q, the damping term
+    and two arrays' worth of tables; with variable density from space order 12
+    the density's two derivative sums.  3D: q, the damping term and the tiled
+    kernel's values, padded to whole tiles (two per point; with variable
+    density the derivative sums and the density too, six), or the z-marching
+    kernel's three derivative sums from space order 12."""
+    npts = int(np.prod(shape))
+    deep = density and space_order >= 12
+    if len(shape) == 2:
+        return (4 + (2 if deep else 0)) * npts * itemsize
+    rows, width = (16, 32) if itemsize == 8 else (8, 64)      # the largest tiles
+    iz, ix, iy = (max(n - space_order, 0) for n in shape)
+    tiles = iz * (-(-ix // rows) * rows) * (-(-iy // width) * width)
+    packed = (6 if density else 2) * tiles
+    return (2 * npts + max(packed, 3 * npts if deep else 0)) * itemsize
+
+
 class DeviceForward:
     """One experiment resident on a GPU.
 
@@ -237,13 +256,11 @@ class DeviceForward:
     @property
     def device_bytes(self):
         """HBM this shot holds while planned: slots, models, shot record and
-        the library's per-point arrays (q, damping term, their copies in tile
-        order and, with variable density, the density's derivative sums and
-        copy)."""
+        the library's per-point arrays."""
         total = sum(t.numel() * t.element_size() for t in self.tensors.values())
         vel = self.tensors["velocity_model"]
-        arrays = 8 if "density_model" in self.tensors else 4
-        return total + arrays * vel.numel() * vel.element_size()
+        return total + library_bytes(tuple(vel.shape), self.kwargs["space_order"],
+                                     vel.element_size(), "density_model" in self.tensors)
 
     @property
     def steps(self):

@@ -36,6 +36,8 @@ from concurrent.futures import Future, ThreadPoolExecutor
 
 import numpy as np
 
+from .device import library_bytes
+
 __all__ = ["ShotServer", "ServeStats", "percentile", "shot_bytes"]
 
 
@@ -48,20 +50,18 @@ def percentile(values, q):
 
 def shot_bytes(solver):
     """HBM an admitted shot holds: wavefield slots, models, shot record and
-    the library's per-point arrays (q, damping term and, in tile order and
-    padded to whole tiles, (dt^2/s)/den and the damping term; with variable
-    density the density's derivative sums and copy too)."""
+    the library's per-point arrays (library_bytes)."""
     if hasattr(solver, "device_bytes"):           # test doubles
         return float(solver.device_bytes)
     sm = solver.space_model
     npts = int(np.prod(sm.extended_shape))
     esz = np.dtype(sm.dtype).itemsize
+    density = sm.density_model is not None
     slots = solver.num_snapshots + 2
-    models = 3 if sm.density_model is not None else 2
-    # variable density in 3D: derivative sums and the density in tile order
-    sums = len(sm.extended_shape) + 1 if sm.density_model is not None else 0
+    models = 3 if density else 2
     rec = solver.time_model.timesteps * solver.receivers.count
-    return float((slots + models + 4 + sums) * npts * esz + rec * esz)
+    return float((slots + models) * npts * esz + rec * esz +
+                 library_bytes(sm.extended_shape, sm.space_order, esz, density))
 
 
 class ServeStats:
