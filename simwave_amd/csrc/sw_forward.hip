@@ -15,6 +15,7 @@
 // slots of HBM, and the even-stride content exchange becomes a swap of the two
 // device pointers.
 #include "sw_kernels.hpp"
+#include "sw_launch.hpp"
 #include "sw_memory.hpp"
 #include "sw_step3d.hpp"
 #include "sw_adjoint.hpp"
@@ -436,6 +437,7 @@ void setup_tiling(Prepared &pr, DeviceArena &arena, hipStream_t st,
 bool prefer_zmarch(const Prepared &pr);
 bool prefer_tiled_vd(const Prepared &pr, bool oblong, const DeviceArena &arena);
 void set_lap_div(Prepared &pr);
+void fit_zmarch(Prepared &pr, size_t nrec);
 #else
 bool zmarch_2d(int R);
 #endif
@@ -661,6 +663,7 @@ Prepared prepare(const Args &a, bool dev_models, unsigned flags,
         if (!pr.tiled) {
             pr.zmarch = true;
             pr.zmarch_zlen = std::max(1, std::min(env_int("SIMWAVE_HIP_ZLEN", 8), 256));
+            fit_zmarch(pr, a.nrec);
             set_lap_div(pr);
         }
     }
@@ -694,6 +697,7 @@ Prepared prepare(const Args &a, bool dev_models, unsigned flags,
                 zl /= 2;
         }
         pr.zmarch_zlen = std::max(1, std::min(zl, 256));
+        fit_zmarch(pr, a.nrec);
         set_lap_div(pr);
     }
 #endif
@@ -1119,7 +1123,8 @@ void setup_tiling(Prepared &pr, DeviceArena &arena, hipStream_t st, const sw::Mo
     T.ntiles = T.ncols * T.gz;
     const long long blocks =
         T.order == 1 ? 8ll * T.chunk * T.gz : (long long)T.ntiles;
-    if (blocks >= (1ll << 31))
+    // (a sixteenth of the launch left to the receivers' blocks)
+    if (!sw::launch_fits(blocks + blocks / 16, K.pack.nt))
         return;
     T.nwords = P.nz / 32 + 3;
     const size_t tile_points = (size_t)T.ncols * Iz * T.ty * T.txr;
@@ -1417,6 +1422,18 @@ struct RecStream {
 };
 
 #if SW_DIM == 3
+// z chunks long enough for all blocks of the z-marching kernel to fit one
+// launch (it lays them along one axis; grids of few points along y have many).
+void fit_zmarch(Prepared &pr, size_t nrec)
+{
+    const Params &P = pr.P;
+    const int R = pr.r;
+    const long long columns = (long long)((P.ny - 2 * R + 63) / 64) *
+                              ((P.nx - 2 * R + sw::kZLines - 1) / sw::kZLines);
+    pr.zmarch_zlen = sw::z_chunk_planes(pr.zmarch_zlen, columns, P.nz - 2 * R, 64 * sw::kZLines,
+                                        (long long)(nrec / sw::kRecPerZ) + 1);
+}
+
 // One step of k_step3d_z over the interior.
 void zmarch_launch(const Prepared &pr, const real_t *uc, const real_t *up, real_t *un, int n,
                    hipStream_t st, LaunchTimer tm, sw::RecArgs rec)
@@ -1427,7 +1444,7 @@ void zmarch_launch(const Prepared &pr, const real_t *uc, const real_t *up, real_
     const int gy = (P.nx - 2 * R + sw::kZLines - 1) / sw::kZLines;
     const long long blocks = (long long)gx * gy * ((P.nz - 2 * R + zl - 1) / zl);
     rec.nrb = (rec.nrec + sw::kRecPerZ - 1) / sw::kRecPerZ;
-    if (blocks + rec.nrb >= (1ll << 31))
+    if (!sw::launch_fits(blocks + rec.nrb, 64 * sw::kZLines))
         fail("grid of %lld blocks is too large for one launch", blocks);
     const dim3 grid((unsigned)(blocks + rec.nrb));
     const dim3 block(64, sw::kZLines);
@@ -2667,7 +2684,7 @@ AdjPlan plan_adjoint(Prepared &pr, DeviceArena &arena, hipStream_t st)
     const long long blocks = 8ll * T.chunk * T.gz;
     // 32-bit buffer offsets over the planes a tile touches
     A.tiled = pbytes * (zlen + 2 * R + 1) < (1ll << 31) && P.ny >= sw::kVec16 &&
-              blocks + total / 64 + 1 < (1ll << 31) && !env_flag("SIMWAVE_HIP_UNTILED");
+              sw::launch_fits(blocks + total / 64 + 1, 64) && !env_flag("SIMWAVE_HIP_UNTILED");
     if (!A.tiled)
         return A;
     A.tiled_blocks = (int)blocks;
