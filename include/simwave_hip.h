@@ -193,6 +193,9 @@ int simwave_hip_gather_2d_cd_f32(float *out, const float *small, int ndim,
  * on a second stream (large grids); 8 times every reverse update kernel
  * with HIP events (simwave_hip_last_timings: [4] their summed seconds,
  * [5] their count).
+ * Where an axis starts with a Neumann face and ends with a Dirichlet one, and
+ * its interior is space_order/2 + 1 points, the velocity gradient on that
+ * Dirichlet plane is wrong (the plane is mirrored before it is zeroed).
  * The shot starts from rest: u's three slots are zeroed first, whatever
  * they hold.  Also writes the shot record and leaves u as after a plain
  * forward.  Returns wall seconds, or -1. */
@@ -367,6 +370,9 @@ int simwave_hip_gather_2d_cd_f64(double *out, const double *small, int ndim,
  * on a second stream (large grids); 8 times every reverse update kernel
  * with HIP events (simwave_hip_last_timings: [4] their summed seconds,
  * [5] their count).
+ * Where an axis starts with a Neumann face and ends with a Dirichlet one, and
+ * its interior is space_order/2 + 1 points, the velocity gradient on that
+ * Dirichlet plane is wrong (the plane is mirrored before it is zeroed).
  * The shot starts from rest: u's three slots are zeroed first, whatever
  * they hold.  Also writes the shot record and leaves u as after a plain
  * forward.  Returns wall seconds, or -1. */
@@ -542,6 +548,9 @@ int simwave_hip_gather_2d_vd_f32(float *out, const float *small, int ndim,
  * on a second stream (large grids); 8 times every reverse update kernel
  * with HIP events (simwave_hip_last_timings: [4] their summed seconds,
  * [5] their count).
+ * Where an axis starts with a Neumann face and ends with a Dirichlet one, and
+ * its interior is space_order/2 + 1 points, the velocity gradient on that
+ * Dirichlet plane is wrong (the plane is mirrored before it is zeroed).
  * The shot starts from rest: u's three slots are zeroed first, whatever
  * they hold.  Also writes the shot record and leaves u as after a plain
  * forward.  Returns wall seconds, or -1. */
@@ -717,6 +726,9 @@ int simwave_hip_gather_2d_vd_f64(double *out, const double *small, int ndim,
  * on a second stream (large grids); 8 times every reverse update kernel
  * with HIP events (simwave_hip_last_timings: [4] their summed seconds,
  * [5] their count).
+ * Where an axis starts with a Neumann face and ends with a Dirichlet one, and
+ * its interior is space_order/2 + 1 points, the velocity gradient on that
+ * Dirichlet plane is wrong (the plane is mirrored before it is zeroed).
  * The shot starts from rest: u's three slots are zeroed first, whatever
  * they hold.  Also writes the shot record and leaves u as after a plain
  * forward.  Returns wall seconds, or -1. */
@@ -891,6 +903,9 @@ int simwave_hip_gather_3d_cd_f32(float *out, const float *small, int ndim,
  * on a second stream (large grids); 8 times every reverse update kernel
  * with HIP events (simwave_hip_last_timings: [4] their summed seconds,
  * [5] their count).
+ * Where an axis starts with a Neumann face and ends with a Dirichlet one, and
+ * its interior is space_order/2 + 1 points, the velocity gradient on that
+ * Dirichlet plane is wrong (the plane is mirrored before it is zeroed).
  * The shot starts from rest: u's three slots are zeroed first, whatever
  * they hold.  Also writes the shot record and leaves u as after a plain
  * forward.  Returns wall seconds, or -1. */
@@ -1065,6 +1080,9 @@ int simwave_hip_gather_3d_cd_f64(double *out, const double *small, int ndim,
  * on a second stream (large grids); 8 times every reverse update kernel
  * with HIP events (simwave_hip_last_timings: [4] their summed seconds,
  * [5] their count).
+ * Where an axis starts with a Neumann face and ends with a Dirichlet one, and
+ * its interior is space_order/2 + 1 points, the velocity gradient on that
+ * Dirichlet plane is wrong (the plane is mirrored before it is zeroed).
  * The shot starts from rest: u's three slots are zeroed first, whatever
  * they hold.  Also writes the shot record and leaves u as after a plain
  * forward.  Returns wall seconds, or -1. */
@@ -1240,6 +1258,9 @@ int simwave_hip_gather_3d_vd_f32(float *out, const float *small, int ndim,
  * on a second stream (large grids); 8 times every reverse update kernel
  * with HIP events (simwave_hip_last_timings: [4] their summed seconds,
  * [5] their count).
+ * Where an axis starts with a Neumann face and ends with a Dirichlet one, and
+ * its interior is space_order/2 + 1 points, the velocity gradient on that
+ * Dirichlet plane is wrong (the plane is mirrored before it is zeroed).
  * The shot starts from rest: u's three slots are zeroed first, whatever
  * they hold.  Also writes the shot record and leaves u as after a plain
  * forward.  Returns wall seconds, or -1. */
@@ -1415,6 +1436,9 @@ int simwave_hip_gather_3d_vd_f64(double *out, const double *small, int ndim,
  * on a second stream (large grids); 8 times every reverse update kernel
  * with HIP events (simwave_hip_last_timings: [4] their summed seconds,
  * [5] their count).
+ * Where an axis starts with a Neumann face and ends with a Dirichlet one, and
+ * its interior is space_order/2 + 1 points, the velocity gradient on that
+ * Dirichlet plane is wrong (the plane is mirrored before it is zeroed).
  * The shot starts from rest: u's three slots are zeroed first, whatever
  * they hold.  Also writes the shot record and leaves u as after a plain
  * forward.  Returns wall seconds, or -1. */

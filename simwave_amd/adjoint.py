@@ -17,6 +17,7 @@ only for device memory and the autograd plumbing.
 """
 import ctypes
 import functools
+import warnings
 
 import numpy as np
 
@@ -37,6 +38,23 @@ def _check(solver):
         raise NotImplementedError("the adjoint covers constant density only")
     if solver.time_model.saving_stride != 0:
         raise ValueError("the adjoint needs saving_stride 0")
+
+
+def zeroed_mirror_axes(shape, space_order, boundary):
+    """Axes of an extended grid whose velocity gradient is wrong on the plane of
+    the Dirichlet face at their end.
+
+    A Neumann face at an axis' start mirrors the r = space_order/2 planes behind
+    it before the Dirichlet face at its end zeroes its own.  Where the interior
+    is r+1 points, the last mirrored plane is that one: it has an adjoint, but
+    the wavefields that the gradient differences hold its zero in place of the
+    mirrored value.  (With the faces the other way round the zero comes first
+    and is what is mirrored.)  `boundary`: the codes of the faces (1 Dirichlet,
+    2 Neumann), two per axis.  Wavefields, shot record, wavelet gradient and
+    image are not affected."""
+    r = space_order // 2
+    return [a for a, n in enumerate(shape)
+            if n - 2 * r == r + 1 and list(boundary[2 * a:2 * a + 2]) == [2, 1]]
 
 
 def checkpoint_interval(dev, checkpoint_every=None):
@@ -71,6 +89,12 @@ def _run(dev, rec_adjoint, checkpoint_every, want_wavelet, stream=None, image=Fa
     fn.argtypes = list(dev._argtypes) + [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                          ctypes.c_size_t, ctypes.c_void_p, ctypes.c_uint]
     vel = dev.tensors["velocity_model"]
+    wrong = [] if image else zeroed_mirror_axes(tuple(vel.shape), int(kw["space_order"]),
+                                                [int(c) for c in kw["boundary_condition"]])
+    if wrong:
+        warnings.warn("the velocity gradient is wrong on the Dirichlet plane at the end of axis %s:"
+                      " the Neumann face at its start mirrors that plane before it is zeroed"
+                      % ", ".join(map(str, wrong)), RuntimeWarning, stacklevel=3)
     grad = torch.zeros(vel.shape, dtype=torch.float64, device=dev.device)
     rec = torch.as_tensor(rec_adjoint, device=dev.device).to(vel.dtype).contiguous()
     if tuple(rec.shape) != tuple(dev.tensors["shot_record"].shape):
@@ -115,6 +139,9 @@ def gradient(solver, rec_adjoint, checkpoint_every=None, wavelet_gradient=False,
 
     Returns
     -------
+    (A RuntimeWarning names grids whose velocity gradient is wrong on a
+    plane: zeroed_mirror_axes.)
+
     dict with ``shot_record`` (numpy), ``grad_velocity`` (float64 numpy,
     extended shape) and, with wavelet_gradient, ``grad_wavelet``
     ([timesteps, sources]).

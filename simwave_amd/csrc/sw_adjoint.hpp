@@ -854,6 +854,64 @@ k_adj_update_z2d(Params P, AdjArgs A, int zlen, int gx, int step_blocks)
 }
 #endif
 
+// Velocity derivative of step n on a Dirichlet plane (`face`) whose points have
+// an adjoint: an earlier boundary phase mirrors the plane before its own zeroes
+// it, and a receiver box holds the mirrored values.  The levels are zero there,
+// so the update's step difference adds nothing; what the step added before the
+// zero is formed here, l^k dc (L u^n + s).  Rare and small (one plane, few
+// points with l != 0): a launch of its own, one thread per point.  planes: all
+// faces so treated; a point on several is the first one's.
+__global__ void __launch_bounds__(256)
+k_adj_zeroed_plane(Params P, const real_t *__restrict__ vel, const real_t *__restrict__ l,
+                   const real_t *__restrict__ u, real_t *__restrict__ gacc, int face,
+                   unsigned planes, int n)
+{
+    const int r = P.r, axis = face >> 1;
+    const int N[3] = {P.nz, P.nx, SW_DIM == 3 ? P.ny : 1};
+    int x[3] = {0, 0, 0};
+    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+#pragma unroll
+    for (int a = SW_DIM - 1; a >= 0; a--) {
+        if (a == axis)
+            continue;
+        const int len = N[a] - 2 * r;
+        x[a] = r + (int)(t % len);
+        t /= len;
+    }
+    if (t != 0)
+        return;
+    x[axis] = face & 1 ? N[axis] - r - 1 : r;
+    for (int f = 0; f < face; f++)
+        if ((planes >> f & 1) && x[f >> 1] == (f & 1 ? N[f >> 1] - r - 1 : r))
+            return;
+    const long long p = (long long)x[0] * P.sz + (long long)x[1] * P.sx + x[2];
+    const real_t lv = l[p];
+    if (lv == (real_t)0)
+        return;
+    const long long st[3] = {P.sz, P.sx, 1};
+    const double h2[3] = {(double)P.dz2, (double)P.dx2, (double)P.dy2};
+    double term = 0;
+#pragma unroll
+    for (int a = 0; a < SW_DIM; a++) {
+        double acc = (double)P.c2[0] * (double)u[p];
+        for (int m = 1; m <= r; m++)
+            acc += (double)P.c2[m] * ((double)u[p + m * st[a]] + (double)u[p - m * st[a]]);
+        term += acc / h2[a];
+    }
+    for (int s = 0; s < P.nsrc; s++) {
+        const Box b = P.sbox[s];
+        bool in = true;
+#pragma unroll
+        for (int a = 0; a < SW_DIM; a++)
+            in = in && x[a] >= b.lo[a] && x[a] <= b.hi[a];
+        if (in)
+            term += (double)box_weight(b, P.sw, x[0], x[1], x[2]) * (double)wavelet_amp(P, n, s);
+    }
+    const double den = 1.0 + (double)P.e[p];
+    const double dc = 2.0 * (double)P.q[p] / ((double)vel[p] * den * den);
+    gacc[p] += (real_t)((double)lv * dc * term);
+}
+
 // Wavelet gradient of step n (k = n+1): gw[s] = sum_p kws_{s,p} c_p ub_p
 // (c = q / den) over the source box's interior points, in float64, one
 // block per source.  (The velocity derivative of the source term is part

@@ -2631,6 +2631,31 @@ int adj_zlen_2d(const Params &P, int R)
 #endif
 
 #if !SW_VD
+// Dirichlet faces (bits) whose planes take their velocity derivative from
+// k_adj_zeroed_plane: those a receiver box holds together with the halo of a
+// Neumann face of a later axis, whose phase mirrors the plane before this one
+// zeroes it.  An axis of r+1 interior points that starts with a Neumann face is
+// left out: there the stencil reads the mirrored plane too, and its gradient
+// stays what it always was (the Python caller is warned).
+unsigned zeroed_planes(const Params &P, const std::vector<Box> &rec)
+{
+    const int r = P.r, N[3] = {P.nz, P.nx, SW_DIM == 3 ? P.ny : 1};
+    unsigned planes = 0;
+    for (int f = 0; f < 2 * SW_DIM; f++) {
+        const int a = f / 2, p = f & 1 ? N[a] - r - 1 : r;
+        if (P.bc[f] != 1 || (P.bc[f & ~1] == 2 && N[a] - 2 * r == r + 1))
+            continue;
+        for (int g = 2 * (a + 1); g < 2 * SW_DIM; g++)
+            for (size_t q = 0; q < rec.size() && P.bc[g] == 2; q++) {
+                const Box &b = rec[q];
+                const bool halo = g & 1 ? b.hi[g / 2] >= N[g / 2] - r : b.lo[g / 2] < r;
+                if (halo && b.lo[a] <= p && p <= b.hi[a])
+                    planes |= 1u << f;
+            }
+    }
+    return planes;
+}
+
 // Launch shape of the reverse updates of one gradient.
 struct AdjPlan {
     unsigned halo_lines = 0;    // lines of the Neumann faces, in face order
@@ -2903,6 +2928,10 @@ double run_adjoint(const Args &a, const real_t *rec_adj, double *grad, real_t *g
         fail("the adjoint needs every source box inside the interior");
     const RecGather rg = build_rec_gather(a, pr, arena, st);
     const Params &P = pr.P;
+    const unsigned planes =
+        image ? 0u
+              : zeroed_planes(P, make_boxes("receiver", a.nrec, a.rint, a.rint_size, a.roff,
+                                            a.rvals_size, dims));
     const size_t npts = (size_t)pr.npts;
     const size_t T = a.n1;
     // K >= T: every level stays in HBM (no checkpoints, no recomputation)
@@ -3053,6 +3082,11 @@ double run_adjoint(const Args &a, const real_t *rec_adj, double *grad, real_t *g
             if (a.nsrc && gw)
                 hipLaunchKernelGGL(sw::k_adj_sources, dim3((unsigned)a.nsrc), dim3(256), 0, st,
                                    P, l, gw + (n - 1) * a.nsrc);
+            for (int f = 0; f < 2 * SW_DIM; f++)
+                if (planes >> f & 1)
+                    hipLaunchKernelGGL(sw::k_adj_zeroed_plane,
+                                       dim3((unsigned)((lines[f / 2] + 255) / 256)), dim3(256), 0,
+                                       st, P, a.vel, l, level_ptr(n), gacc, f, planes, (int)n);
             LaunchTimer tm;
             if (utime.used + 2 <= utime.ev.size()) {
                 tm = LaunchTimer{utime.ev[utime.used], utime.ev[utime.used + 1]};
