@@ -1067,10 +1067,6 @@ TiledKernel tiled_kernel(int R, int v)
     }
 }
 
-// Blocks along y of a launch whose blocks share n planes: a launch takes 65536
-// at most (the device's grid limit along y), and a grid may be deeper.
-unsigned grid_y(int n) { return (unsigned)std::min(n, 65536); }
-
 // Chooses the tile grid and launch order, marks the tile planes that hold
 // damping and packs the coefficients.  Leaves pr.tiled false when the grid
 // does not fit the kernel's 32-bit buffer offsets.  M: the models on the
@@ -1153,7 +1149,7 @@ void setup_tiling(Prepared &pr, DeviceArena &arena, hipStream_t st, const sw::Mo
     }
     T.dmask = mask;
     hipLaunchKernelGGL(M ? sw::k_damp_flags<true> : sw::k_damp_flags<false>,
-                       dim3(T.ncols, grid_y(P.nz)), dim3(256), 0, st, P,
+                       sw::plane_grid(T.ncols, P.nz), dim3(256), 0, st, P,
                        M ? *M : sw::Models{}, P.nz, P.nx, P.ny, R, T.gk, T.ty, T.txr, T.nwords,
                        mask, mask + words - 1);
     hip_check(hipGetLastError(), "k_damp_flags launch");
@@ -1164,7 +1160,7 @@ void setup_tiling(Prepared &pr, DeviceArena &arena, hipStream_t st, const sw::Mo
     real_t *pk = arena.alloc<real_t>(tile_points * (SW_VD ? 5 : 1));
     real_t *pe = arena.alloc<real_t>(tile_points);
     hipLaunchKernelGGL(M ? sw::k_pack_tiles<true> : sw::k_pack_tiles<false>,
-                       dim3(T.ncols, grid_y(Iz)), dim3(256), 0, st, P, M ? *M : sw::Models{}, R,
+                       sw::plane_grid(T.ncols, Iz), dim3(256), 0, st, P, M ? *M : sw::Models{}, R,
                        K.pack, T.gk, T.ty, T.txr, T.ncols, SW_VD, pk, pe);
     hip_check(hipGetLastError(), "k_pack_tiles launch");
     pr.pk = pk;
@@ -2719,7 +2715,7 @@ AdjPlan plan_adjoint(Prepared &pr, DeviceArena &arena, hipStream_t st)
                        dim3((unsigned)std::min<long long>((words + 255) / 256, 4096)), dim3(256),
                        0, st, mask, words);
     T.dmask = mask;
-    hipLaunchKernelGGL(sw::k_damp_flags<false>, dim3(T.ncols, grid_y(P.nz)), dim3(256), 0, st, P,
+    hipLaunchKernelGGL(sw::k_damp_flags<false>, sw::plane_grid(T.ncols, P.nz), dim3(256), 0, st, P,
                        sw::Models{}, P.nz, P.nx, P.ny, R, T.gk, T.ty, T.txr, T.nwords, mask,
                        mask + words - 1);
     hip_check(hipGetLastError(), "k_damp_flags launch");

@@ -100,36 +100,49 @@ __device__ __forceinline__ real_t point_e(const Params &P, const Models &M, long
     return RAW ? prepared_e(M.vel[p], M.damp[p], M.dt) : P.e[p];
 }
 
-// Marks tile planes holding a non-zero damping term.  grid (ncols, any: its
-// blocks share the planes); the mask words must be zeroed beforehand.
+// The z plane of a block of a launch with one block per column and plane
+// (plane_grid: a grid may hold more planes than a launch takes blocks along y).
+__device__ __forceinline__ int plane_of_block()
+{
+    return (int)(blockIdx.z * gridDim.y + blockIdx.y);
+}
+inline dim3 plane_grid(int columns, int planes)
+{
+    constexpr int most = 32768;
+    return dim3((unsigned)columns, (unsigned)(planes < most ? planes : most),
+                (unsigned)((planes + most - 1) / most));
+}
+
+// Marks tile planes holding a non-zero damping term.  plane_grid(ncols, nz);
+// the mask words must be zeroed beforehand.
 template <bool RAW>
 __global__ void __launch_bounds__(256)
 k_damp_flags(Params P, Models M, int nz, int nx, int ny, int R, int gk,
              int ty, int txr, int nwords, unsigned *__restrict__ mask,
              unsigned *__restrict__ den_bad)
 {
-    const int col = blockIdx.x;
+    const int col = blockIdx.x, z = plane_of_block();
+    if (z >= nz)
+        return;
     const int kt = col % gk, jt = col / gk;
     const int k0 = R + kt * ty, j0 = R + jt * txr;
-    for (int z = blockIdx.y; z < nz; z += gridDim.y) {
-        int any = 0;
-        for (int t = threadIdx.x; t < ty * txr; t += blockDim.x) {
-            const int k = k0 + t % ty, j = j0 + t / ty;
-            if (k < ny && j < nx) {
-                const real_t v = point_e<RAW>(P, M, ((long long)z * nx + j) * ny + k);
-                if (v != (real_t)0) {
-                    const double den = fabs((double)(real_t)(1.0 + (double)v));
-                    any |= den >= 0x1p-60 && den <= 0x1p60 ? 1 : 3;
-                }
+    int any = 0;
+    for (int t = threadIdx.x; t < ty * txr; t += blockDim.x) {
+        const int k = k0 + t % ty, j = j0 + t / ty;
+        if (k < ny && j < nx) {
+            const real_t v = point_e<RAW>(P, M, ((long long)z * nx + j) * ny + k);
+            if (v != (real_t)0) {
+                const double den = fabs((double)(real_t)(1.0 + (double)v));
+                any |= den >= 0x1p-60 && den <= 0x1p60 ? 1 : 3;
             }
         }
-        const int damped = __syncthreads_or(any);
-        const int bad = __syncthreads_or(any & 2);
-        if (threadIdx.x == 0 && damped) {
-            atomicOr(&mask[(long long)col * nwords + (z >> 5)], 1u << (z & 31));
-            if (bad)
-                atomicOr(den_bad, 1u);
-        }
+    }
+    const int damped = __syncthreads_or(any);
+    const int bad = __syncthreads_or(any & 2);
+    if (threadIdx.x == 0 && damped) {
+        atomicOr(&mask[(long long)col * nwords + (z >> 5)], 1u << (z & 31));
+        if (bad)
+            atomicOr(den_bad, 1u);
     }
 }
 
@@ -158,36 +171,37 @@ k_pack_tiles(Params P, Models M, int R, PackShape S, int gk, int ty, int txr, in
     const int lp = S.rpt * S.v, nc = lp / kVec16, na = rho ? 5 : 1;
     const int tp = S.nt * lp;                       // points of a tile plane
     const int npl = P.nz - 2 * R;
-    const int col = blockIdx.x;
+    const int col = blockIdx.x, z = plane_of_block();
+    if (z >= npl)
+        return;
     const int k0 = R + col % gk * ty, j0 = R + col / gk * txr;
-    for (int z = blockIdx.y; z < npl; z += gridDim.y)
-        for (int t = threadIdx.x; t < tp; t += blockDim.x) {
-            const int x = t % kVec16, tid = t / kVec16 % S.nt, c = t / kVec16 / S.nt;
-            const int l = c * kVec16 + x, lane = tid % 64, lw = 64 / S.wr;
-            const int slot = tid / 64 * S.wr + lane / lw;
-            const int j = j0 + slot * S.rpt + l / S.v;
-            const int k = k0 + lane % lw * S.v + l % S.v;
-            const int i = R + z;
-            real_t v[5] = {0, 0, 0, 0, 0}, e = 0;
-            if (j < P.nx - R && k < P.ny - R) {
-                const long long p = (long long)i * P.sz + (long long)j * P.sx + k;
-                e = point_e<RAW>(P, M, p);
-                v[0] = point_q<RAW>(P, M, p) / (real_t)(1.0 + (double)e);
-                if (rho) {
-                    const real_t *__restrict__ d = P.rho + p;
-                    for (int m = 1; m <= R; m++) {
-                        v[1] += P.c1[m] * (d[m * P.sz] - d[-m * P.sz]);
-                        v[2] += P.c1[m] * (d[m * P.nx] - d[-m * P.nx]);
-                        v[3] += P.c1[m] * (d[m] - d[-m]);
-                    }
-                    v[4] = d[0];
+    for (int t = threadIdx.x; t < tp; t += blockDim.x) {
+        const int x = t % kVec16, tid = t / kVec16 % S.nt, c = t / kVec16 / S.nt;
+        const int l = c * kVec16 + x, lane = tid % 64, lw = 64 / S.wr;
+        const int slot = tid / 64 * S.wr + lane / lw;
+        const int j = j0 + slot * S.rpt + l / S.v;
+        const int k = k0 + lane % lw * S.v + l % S.v;
+        const int i = R + z;
+        real_t v[5] = {0, 0, 0, 0, 0}, e = 0;
+        if (j < P.nx - R && k < P.ny - R) {
+            const long long p = (long long)i * P.sz + (long long)j * P.sx + k;
+            e = point_e<RAW>(P, M, p);
+            v[0] = point_q<RAW>(P, M, p) / (real_t)(1.0 + (double)e);
+            if (rho) {
+                const real_t *__restrict__ d = P.rho + p;
+                for (int m = 1; m <= R; m++) {
+                    v[1] += P.c1[m] * (d[m * P.sz] - d[-m * P.sz]);
+                    v[2] += P.c1[m] * (d[m * P.nx] - d[-m * P.nx]);
+                    v[3] += P.c1[m] * (d[m] - d[-m]);
                 }
+                v[4] = d[0];
             }
-            const long long plane = (long long)col * npl + z;
-            for (int a = 0; a < na; a++)
-                pk[((plane * na + a) * nc + c) * (S.nt * kVec16) + tid * kVec16 + x] = v[a];
-            pe[(plane * nc + c) * (S.nt * kVec16) + tid * kVec16 + x] = e;
         }
+        const long long plane = (long long)col * npl + z;
+        for (int a = 0; a < na; a++)
+            pk[((plane * na + a) * nc + c) * (S.nt * kVec16) + tid * kVec16 + x] = v[a];
+        pe[(plane * nc + c) * (S.nt * kVec16) + tid * kVec16 + x] = e;
+    }
 }
 
 // Bits z0 .. z0+63 of a tile column's damping mask.
