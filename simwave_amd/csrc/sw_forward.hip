@@ -805,18 +805,18 @@ void set_lap_div(Prepared &pr)
 // density: radius 4 (space order 8) carries every configuration, other radii
 // 0, 4, 8, 17 and 18; SIMWAVE_HIP_TILE picks one, otherwise default_tile().
 // Variable density carries one shape per radius (tiled_entry).
-// Measured per launch on one MI355X with the packed coefficients:
+// Measured per launch on one MI355X, receivers inside, 20 damping cells a side:
 //  * float32 radius 4: 8 rows x 64 points of 8-byte lanes with 4 rows per
-//    lane (17) for large grids (472^3: 502 us, the same tile of 16-byte lanes
-//    with 2 rows per lane (10) 526; 216 x 316 x 316 interior: 136 each), the
-//    16-byte tile below 20 M interior points (240^3: 88 against 90 us).
-//  * float32 radius 3: 17 (340^3: 228 us, 8: 252).  Radii 5-10: 8 rows x 32
-//    points of 16-byte lanes (8): 240^3 so16 97 us (17: 107), so20 116 (122);
-//    241 x 317 x 341 so12 176 (174).
+//    lane (17) for large grids (472^3 with 40 cells: 485 us, the same tile of
+//    16-byte lanes with 2 rows per lane (10) 503; 216 x 316 x 316 interior: 128
+//    and 134), the 16-byte tile below 20 M interior points (240^3: 90, 17 88).
+//  * float32 radius 3: 17 (340^3: 233 us, 8: 274).  Radii 5-10: 8 rows x 32
+//    points of 16-byte lanes (8): 240^3 so16 103 us (17: 117), so20 129 (133);
+//    241 x 317 x 341 so12 186 (175).
 //  * float64: radius 4 the 16-byte 8 x 32 tile (10: 221 x 243 x 259 152 us, 17
-//    153, 8 173); below, 8 x 16 points with 2 rows per lane (18: 240^3 so4
-//    142, 17 147, 4 158); radii 5-7 four wavefronts (4: so12 157, 8 175);
-//    above, one (8: so16 168, 4 176).
+//    151, 8 175); below, 4 x 32 points with 2 rows per lane (18: 240^3 so4
+//    142, 17 149, 4 170); radii 5-7 four wavefronts (4: so12 171, 8 184);
+//    above, one (8: so16 176, 4 183).
 constexpr int kTileShapes = 24;
 // scratch left to the small tables behind the packed coefficients
 constexpr size_t kPackSlack = 1u << 20;
@@ -832,11 +832,11 @@ int default_tile(int R, bool div64, long long interior)
 }
 
 // Planes per z chunk.  Short chunks: the tiles in flight on an XCD then cover
-// few planes and share their halo rows in its L2 (256^3 variable density so8:
-// 4 planes fetch 0.82 GB per step and take 185 us, 12 planes 212 us, 24
+// few planes and share their halo rows in its L2 (276^3 variable density so8:
+// 4 planes fetch 0.82 GB per step and take 183 us, 12 planes 203 us, 24
 // planes 1.02 GB); large grids and the long prologues of high orders want a
-// few more (472^3: 6 planes 502 us, 4 514; so16 float64 240^3: 12 planes 168,
-// 4 178), small grids fewer, to fill the chip: below 1 M interior points 2
+// few more (472^3: 6 planes 485 us, 4 538; so16 float64 240^3: 12 planes 176,
+// 4 196), small grids fewer, to fill the chip: below 1 M interior points 2
 // planes everywhere (56^3 so10 12.8 us, 4 planes 19.8; 53^3 float64 so16 9.9
 // and 13.4), up to 5 M still 2 for float32 up to radius 8 and for constant
 // density in float64 up to radius 3 (150^3 so12 32.1, 4 planes 33.0; 150^3
@@ -873,10 +873,12 @@ long long interior_points(const Prepared &pr)
 // tiles to keep the tiled kernel's 2 per SIMD busy; its neighbour reads
 // through the caches lose once there are plenty.  Measured per launch
 // (float32, cubes of the interior size): radius 1-2 at every size (340^3 so2:
-// 203 against 235 us, so4 235 against 243); radius 3 (340^3) 255 against 228;
-// radius 4 168^3 41 against 46 us, 240^3 100 against 88, 216 x 316 x 316 148
-// against 136; radius 5+ never (its register queue is 2R+1 deep).  Float64:
-// the tiled kernel (240^3 so4: 155 against 142 us; so8 229 against 152).
+// 195 against 237 us, so4 221 against 247); radius 3 (340^3) 239 against 233;
+// radius 4 168^3 38 against 46 us, 240^3 96 against 88, 216 x 316 x 316 140
+// against 128; radius 5+ never (its register queue is 2R+1 deep).  Float64:
+// the tiled kernel (240^3 so4: 149 against 142 us, so6 180 against 144, 221 x
+// 243 x 259 so8 219 against 152; so2 alone is the z-marching kernel's, 132
+// against 156).
 // Variable density, where the tiled kernel does not run: float32 always,
 // 1.2-1.8x faster than the LDS-tiled k_step3d (176^3-448^3, orders 2-16);
 // float64 at radius <= 4, above which its double-precision register queues
@@ -891,15 +893,15 @@ bool prefer_zmarch(const Prepared &pr)
 }
 
 // Variable density: whether the tiled kernel runs.  Always where nx != ny
-// (only it has the reference's x-axis stride; 160 x 200 x 271 so4: 92 us for
-// the whole step, the generic kernels 85 us for the stencil alone and 22 us
-// for sources and boundaries; so16 160 against 232 us).  Otherwise from 2 M
-// interior points on: float32 from radius 3 (276^3 so8: 185 us, z-marching
-// 275; so16 220 against 317; 148^3 so8 38 against 54; 116^3 29 against 30;
-// but 220^3 so2 100 against 80), radius 2 from 12 M points (240^3 so4 128
-// against 133, 276^3 184 against 196; 220^3 104 against 105), float64 from
-// radius 2 (220^3 so4 170 against 227, so8 171 against 344, so16 234 against
-// k_step3d's 459).  A caller-owned arena (the allocation-free entry) has no room
+// (only it has the reference's x-axis stride; 160 x 200 x 271 so4: 90 us for
+// the whole step, the generic kernels 81 us for the stencil alone and 22 us
+// for sources and boundaries; so16 177 against 214 us).  Otherwise from 2 M
+// interior points on: float32 from radius 3 (276^3 so8: 184 us, z-marching
+// 250; so16 230 against 284; 148^3 so8 33 against 50; 116^3 22 against 27;
+// but 220^3 so2 97 against 73), radius 2 from 12 M points (240^3 so4 125
+// against 131, 276^3 186 against 195; 220^3 102 against 99), float64 from
+// radius 2 (220^3 so4 161 against 210, so8 175 against 321, so16 257 against
+// k_step3d's 465; all with 20 damping cells a side).  A caller-owned arena (the allocation-free entry) has no room
 // for the packed coefficients.
 bool prefer_tiled_vd(const Prepared &pr, bool oblong, const DeviceArena &arena)
 {
@@ -1931,17 +1933,28 @@ double run_host(const Args &a, bool lean)
         std::vector<real_t *> phys(a.num_snapshots, nullptr);
         std::vector<real_t *> pool;
         std::map<real_t *, hipEvent_t> free_after;   // buffer -> download done
+        // slots that hold a step's output, and whether one of them has gone to
+        // the caller: from then on the run cannot start over
+        std::vector<char> output(a.num_snapshots, 0);
+        bool delivered = false;
         auto acquire = [&]() -> real_t * {
-            if (pool.empty())
-                return arena.alloc<real_t>(npts);
-            real_t *p = pool.back();
-            pool.pop_back();
-            auto it = free_after.find(p);
-            if (it != free_after.end()) {
-                hip_check(hipStreamWaitEvent(st, it->second, 0), "hipStreamWaitEvent");
-                free_after.erase(it);
+            if (!pool.empty()) {
+                real_t *p = pool.back();
+                pool.pop_back();
+                auto it = free_after.find(p);
+                if (it != free_after.end()) {
+                    hip_check(hipStreamWaitEvent(st, it->second, 0), "hipStreamWaitEvent");
+                    free_after.erase(it);
+                }
+                return p;
             }
-            return p;
+            try {
+                return arena.alloc<real_t>(npts);
+            } catch (const OutOfMemory &e) {
+                if (delivered)
+                    throw Failure(e);
+                throw;
+            }
         };
         // bucket slots by the step that uploads / downloads them
         std::vector<std::vector<size_t>> up_at(plan.size()), down_at(plan.size());
@@ -1953,18 +1966,6 @@ double run_host(const Args &a, bool lean)
             down_at[last[sl]].push_back(sl);
             const StepSlots &s = plan[first[sl]];
             any_frame |= s.next == sl && s.prev != sl && s.cur != sl;
-        }
-        // as many buffers as slots are resident at once, before the first
-        // download: a run that finds too little memory has written nothing
-        {
-            size_t resident = 0, most = 0;
-            for (size_t idx = 0; idx < plan.size(); idx++) {
-                resident += up_at[idx].size();
-                most = std::max(most, resident);
-                resident -= down_at[idx].size();
-            }
-            while (pool.size() < most)
-                pool.push_back(arena.alloc<real_t>(npts));
         }
         // halo frame: indices on the device, packed values staged pinned
         std::vector<unsigned long long> fidx;
@@ -2040,10 +2041,15 @@ double run_host(const Args &a, bool lean)
             }
         };
         auto after = [&](size_t idx) {
+            const StepSlots &s = plan[idx];
+            output[s.next] = 1;
+            if (s.swap_after)
+                output[s.swap_a] = output[s.swap_b] = 1;
             if (down_at[idx].empty())
                 return;
             hip_check(hipEventRecord(slot_done, st), "hipEventRecord");
             for (size_t sl : down_at[idx]) {
+                delivered = delivered || output[sl];
                 down.push(phys[sl], a.u + sl * npts, slot_done);
                 // the buffer may be rewritten once its download has fired
                 hipEvent_t e = nullptr;

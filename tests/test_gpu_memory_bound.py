@@ -68,6 +68,25 @@ def test_forward_without_room_for_packed_coefficients(name, monkeypatch):
         dev.run()
 
 
+@pytest.mark.parametrize("stride", [1, 2, 3])
+def test_host_call_that_saves_levels(stride, monkeypatch):
+    """Buffers are taken as slots are first used: the run starts over as long
+    as no output has been returned."""
+    print("bounded host call, stride", stride, flush=True)
+    params = dict(CASES["vd_oblong"], stride=stride)
+    s = sw.Solver(**cases.make_case(dim=3, tf=0.012, damping=20.0, window=3, **params)())
+    s._middleware.verbose = False
+    want = s.forward()
+    # q, e, the density, four slots and the halo frame
+    for arrays in (8, 13):              # without and with some of the packed values
+        monkeypatch.setenv("SIMWAVE_HIP_RUN_MB", bound(s, arrays))
+        for a, b in zip(s.forward(), want):
+            np.testing.assert_array_equal(a, b)
+    monkeypatch.setenv("SIMWAVE_HIP_RUN_MB", bound(s, 4))
+    with pytest.raises(RuntimeError, match="out of memory"):
+        s.forward()
+
+
 @pytest.mark.parametrize("name", ["cd_so12", "cd_f64"])
 def test_gradient_without_room_for_packed_coefficients(name, monkeypatch):
     print("bounded gradient", name, flush=True)
