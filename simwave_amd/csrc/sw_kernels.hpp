@@ -399,8 +399,8 @@ __device__ __forceinline__ void store_with_bc(const Params &P, real_t *un,
 // points at 472^3: 28 us alone per step, 56 before (single loads, the
 // chain waiting for every LDS read).
 // Axis weights kept in LDS per receiver (WC): a wider box reads them from
-// memory.  The step launches' gathers keep 32, the default window's three
-// axes taking 27, for the sake of the step's occupancy.
+// memory.  The tiled steps' gathers keep 32, the default window's three axes
+// taking 27, for the sake of the step's occupancy.
 constexpr int kRecWeights = 64, kRecWeightsStep = 32;
 
 template <int RPB, int CH, int WC = kRecWeights>
@@ -874,11 +874,12 @@ struct RecArgs {
 };
 
 // The z-marching kernels' gather: 16 receivers per block, rounds of 256 (128
-// in float64) products, 20 KB of LDS (22 KB): 8 (7) blocks per CU, as many as
-// the step's registers allow.
+// in float64) products, 22 KB of LDS (26 KB).  A block is 8 wavefronts, 2 per
+// SIMD, so a CU holds at most 4: the LDS leaves them room, the step's registers
+// decide.
 constexpr int kRecPerZ = 16;
 constexpr int kRecChunkZ = sizeof(real_t) == 4 ? 256 : 128;
-typedef RecShared<kRecPerZ, kRecChunkZ, kRecWeightsStep> RecZ;
+typedef RecShared<kRecPerZ, kRecChunkZ> RecZ;
 
 // Wavefronts per SIMD asked of the compiler for the radii where it would give
 // the two paths of a launch together a few registers more than the step alone
