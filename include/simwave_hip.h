@@ -157,7 +157,7 @@ int simwave_hip_plan_destroy_2d_cd_f32(void *plan);
  * enqueues up to `steps` further steps of each of the `count` plans on
  * `stream`, after each plan's earlier work.  Plans that can be batched
  * (simwave_hip_plan_batchable_2d_cd_f32) advance together, radius by radius:
- * one step kernel and one receiver kernel per time step for all of them
+ * one kernel per time step takes the steps and receivers of all of them
  * (up to 48 per launch); the others run as simwave_hip_plan_run_2d_cd_f32.
  * left[i] receives plan i's remaining steps.  Returns 0, or -1. */
 int simwave_hip_plans_run_2d_cd_f32(void **plans, int count, size_t steps,
@@ -334,7 +334,7 @@ int simwave_hip_plan_destroy_2d_cd_f64(void *plan);
  * enqueues up to `steps` further steps of each of the `count` plans on
  * `stream`, after each plan's earlier work.  Plans that can be batched
  * (simwave_hip_plan_batchable_2d_cd_f64) advance together, radius by radius:
- * one step kernel and one receiver kernel per time step for all of them
+ * one kernel per time step takes the steps and receivers of all of them
  * (up to 48 per launch); the others run as simwave_hip_plan_run_2d_cd_f64.
  * left[i] receives plan i's remaining steps.  Returns 0, or -1. */
 int simwave_hip_plans_run_2d_cd_f64(void **plans, int count, size_t steps,
@@ -512,7 +512,7 @@ int simwave_hip_plan_destroy_2d_vd_f32(void *plan);
  * enqueues up to `steps` further steps of each of the `count` plans on
  * `stream`, after each plan's earlier work.  Plans that can be batched
  * (simwave_hip_plan_batchable_2d_vd_f32) advance together, radius by radius:
- * one step kernel and one receiver kernel per time step for all of them
+ * one kernel per time step takes the steps and receivers of all of them
  * (up to 48 per launch); the others run as simwave_hip_plan_run_2d_vd_f32.
  * left[i] receives plan i's remaining steps.  Returns 0, or -1. */
 int simwave_hip_plans_run_2d_vd_f32(void **plans, int count, size_t steps,
@@ -690,7 +690,7 @@ int simwave_hip_plan_destroy_2d_vd_f64(void *plan);
  * enqueues up to `steps` further steps of each of the `count` plans on
  * `stream`, after each plan's earlier work.  Plans that can be batched
  * (simwave_hip_plan_batchable_2d_vd_f64) advance together, radius by radius:
- * one step kernel and one receiver kernel per time step for all of them
+ * one kernel per time step takes the steps and receivers of all of them
  * (up to 48 per launch); the others run as simwave_hip_plan_run_2d_vd_f64.
  * left[i] receives plan i's remaining steps.  Returns 0, or -1. */
 int simwave_hip_plans_run_2d_vd_f64(void **plans, int count, size_t steps,
@@ -867,7 +867,7 @@ int simwave_hip_plan_destroy_3d_cd_f32(void *plan);
  * enqueues up to `steps` further steps of each of the `count` plans on
  * `stream`, after each plan's earlier work.  Plans that can be batched
  * (simwave_hip_plan_batchable_3d_cd_f32) advance together, radius by radius:
- * one step kernel and one receiver kernel per time step for all of them
+ * one kernel per time step takes the steps and receivers of all of them
  * (up to 48 per launch); the others run as simwave_hip_plan_run_3d_cd_f32.
  * left[i] receives plan i's remaining steps.  Returns 0, or -1. */
 int simwave_hip_plans_run_3d_cd_f32(void **plans, int count, size_t steps,
@@ -1044,7 +1044,7 @@ int simwave_hip_plan_destroy_3d_cd_f64(void *plan);
  * enqueues up to `steps` further steps of each of the `count` plans on
  * `stream`, after each plan's earlier work.  Plans that can be batched
  * (simwave_hip_plan_batchable_3d_cd_f64) advance together, radius by radius:
- * one step kernel and one receiver kernel per time step for all of them
+ * one kernel per time step takes the steps and receivers of all of them
  * (up to 48 per launch); the others run as simwave_hip_plan_run_3d_cd_f64.
  * left[i] receives plan i's remaining steps.  Returns 0, or -1. */
 int simwave_hip_plans_run_3d_cd_f64(void **plans, int count, size_t steps,
@@ -1222,7 +1222,7 @@ int simwave_hip_plan_destroy_3d_vd_f32(void *plan);
  * enqueues up to `steps` further steps of each of the `count` plans on
  * `stream`, after each plan's earlier work.  Plans that can be batched
  * (simwave_hip_plan_batchable_3d_vd_f32) advance together, radius by radius:
- * one step kernel and one receiver kernel per time step for all of them
+ * one kernel per time step takes the steps and receivers of all of them
  * (up to 48 per launch); the others run as simwave_hip_plan_run_3d_vd_f32.
  * left[i] receives plan i's remaining steps.  Returns 0, or -1. */
 int simwave_hip_plans_run_3d_vd_f32(void **plans, int count, size_t steps,
@@ -1400,7 +1400,7 @@ int simwave_hip_plan_destroy_3d_vd_f64(void *plan);
  * enqueues up to `steps` further steps of each of the `count` plans on
  * `stream`, after each plan's earlier work.  Plans that can be batched
  * (simwave_hip_plan_batchable_3d_vd_f64) advance together, radius by radius:
- * one step kernel and one receiver kernel per time step for all of them
+ * one kernel per time step takes the steps and receivers of all of them
  * (up to 48 per launch); the others run as simwave_hip_plan_run_3d_vd_f64.
  * left[i] receives plan i's remaining steps.  Returns 0, or -1. */
 int simwave_hip_plans_run_3d_vd_f64(void **plans, int count, size_t steps,
